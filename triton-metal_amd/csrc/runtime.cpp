@@ -53,6 +53,14 @@
 #define TM_FWD_FAST_THREADS 256
 #endif
 
+/* Fewest 128-row workgroups for which the padded 16-bit attention kernels run
+ * (forward + backward, bf16 causal: 4 heads of 128 rows at head_dim 80 26 us
+ * against the generic kernels' 74; one head of 300 rows keeps the generic
+ * kernels' ranges) */
+#ifndef TM_ATTN_PAD_MIN
+#define TM_ATTN_PAD_MIN 4
+#endif
+
 namespace {
 
 /* ---- errors ----------------------------------------------------------------
@@ -573,21 +581,59 @@ bool fast_paths_enabled() {
   return enabled;
 }
 
-/* The specialised attention kernels need a 16-bit element type, head_dim 64
- * or 128, 16-byte aligned rows and a positive finite scale. */
-/* The fast kernels copy K/V/Q/dO tiles through a buffer resource based at a
- * head's first row: a head's rows must span fewer than 2^31 bytes. */
-bool attn_fast_ok(const BuiltinSpec &spec, int32_t stride_head, int32_t stride_seq,
-                  int32_t n_ctx, float sm_scale) {
+/* The 16-bit MFMA attention kernels need a 16-bit element type, 16-byte
+ * aligned rows and a positive finite scale.  They copy K/V/Q/dO tiles through
+ * a buffer resource based at a head's first row: a head's rows must span fewer
+ * than 2^31 bytes. */
+bool attn_half_ok(const BuiltinSpec &spec, int32_t stride_head, int32_t stride_seq, int32_t n_ctx,
+                  float sm_scale) {
   const int64_t head_bytes =
       ((int64_t)(n_ctx > 0 ? n_ctx - 1 : 0) * stride_seq + spec.head_dim) * 2;
-  return fast_paths_enabled() && spec.element != Element::F32 &&
-         (spec.head_dim == 64 || spec.head_dim == 128) && stride_seq % 8 == 0 &&
+  return fast_paths_enabled() && spec.element != Element::F32 && stride_seq % 8 == 0 &&
          stride_head % 8 == 0 && std::isfinite(sm_scale) && sm_scale > 0.f &&
          head_bytes <= INT32_MAX;
 }
 
+/* head_dim 64 and 128 run the specialised kernels (attn_fast.hip) */
+bool attn_fast_ok(const BuiltinSpec &spec, int32_t stride_head, int32_t stride_seq,
+                  int32_t n_ctx, float sm_scale) {
+  return (spec.head_dim == 64 || spec.head_dim == 128) &&
+         attn_half_ok(spec, stride_head, stride_seq, n_ctx, sm_scale);
+}
+
+/* Other head dimensions that are multiples of 8 run the same kernels padded
+ * (attn_pad.hip), contracted at this many columns; 0: the generic kernels.
+ * Their workgroups take 128 rows and do not split into ranges, so the smallest
+ * grids stay with the generic kernels, whose ranges fill the chip. */
+int attn_pad_width(const BuiltinSpec &spec, int64_t heads, int32_t stride_head, int32_t stride_seq,
+                   int32_t n_ctx, float sm_scale) {
+  const int d = spec.head_dim;
+  if (d == 64 || d == 128 || d % 8 || cdiv(n_ctx, 128) * heads < TM_ATTN_PAD_MIN ||
+      !attn_half_ok(spec, stride_head, stride_seq, n_ctx, sm_scale))
+    return 0;
+  /* one long head at 32 columns: the generic kernels' ranges win (1 x 2000 at
+   * head_dim 32: 72 against 91 us; 2 x 1000: 58 against 54) */
+  if (d <= 32 && heads == 1 && n_ctx > 512) return 0;
+  return d <= 32 ? 32 : d <= 64 ? 64 : d <= 80 ? 80 : d <= 96 ? 96 : 128;
+}
+
 int padded_head_dim(int d) { return d <= 32 ? 32 : d <= 64 ? 64 : d <= 96 ? 96 : 128; }
+
+/* Delta on the padded kernel, 256 rows to a workgroup: at the 128-column pitch
+ * (164 registers) only with a workgroup for every compute unit (head_dim 80,
+ * 32 heads of 1000 rows: 6.0 against the generic kernel's 5.4 us; 64 heads 6.1
+ * against 7.3, 128 heads of 4000 27 against 42), at the 64-column pitch always
+ * (head_dim 32: 3.7 against 4.1 and 12 against 22 us). */
+int attn_pre_pad_width(const BuiltinSpec &spec, int64_t heads, int32_t stride_head,
+                       int32_t stride_seq, int32_t n_ctx) {
+  const int width = attn_pad_width(spec, heads, stride_head, stride_seq, n_ctx, 1.f);
+  return width <= 64 || cdiv(n_ctx, 256) * heads >= device().compute_units ? width : 0;
+}
+
+std::string attn_pad_symbol(const char *op, const BuiltinSpec &spec, int width) {
+  return format("tm_attn_%s_generic_%s_p%d%s", op, element_name(spec.element), width,
+                spec.causal ? "_causal" : "");
+}
 
 std::string attn_symbol(const char *op, const BuiltinSpec &spec) {
   return format("tm_attn_%s_generic_%s_d%d%s", op, element_name(spec.element),
@@ -1018,6 +1064,11 @@ Plan plan_builtin(Kernel &k, const Library &lib, const std::vector<Arg> &args, i
                               spec.causal ? "_causal" : "");
         plan.grid[0] = (unsigned)(cdiv(p.n_ctx, TM_FWD_FAST_ROWS) * heads);
         plan.block = TM_FWD_FAST_THREADS;
+      } else if (const int width = attn_pad_width(spec, heads, p.stride_head, p.stride_seq,
+                                                  p.n_ctx, p.sm_scale)) {
+        plan.variant = attn_pad_symbol("fwd", spec, width);
+        plan.grid[0] = (unsigned)(cdiv(p.n_ctx, TM_FWD_FAST_ROWS) * heads);
+        plan.block = TM_FWD_FAST_THREADS;
       } else {
         plan.variant = attn_symbol("fwd", spec);
         plan.grid[0] = (unsigned)cdiv(p.n_ctx, 64);
@@ -1083,6 +1134,10 @@ Plan plan_builtin(Kernel &k, const Library &lib, const std::vector<Arg> &args, i
       if (attn_fast_ok(spec, p.stride_head, p.stride_seq, p.n_ctx, 1.f)) {
         plan.variant = format("tm_attn_pre_fast_%s_d%d", el, spec.head_dim);
         plan.grid[0] = (unsigned)(cdiv(p.n_ctx, 256) * heads);
+      } else if (const int width =
+                     attn_pre_pad_width(spec, heads, p.stride_head, p.stride_seq, p.n_ctx)) {
+        plan.variant = format("tm_attn_pre_generic_%s_p%d", el, width <= 64 ? 64 : 128);
+        plan.grid[0] = (unsigned)(cdiv(p.n_ctx, 256) * heads);
       } else {
         plan.variant = format("tm_attn_pre_generic_%s", el);
         plan.grid[0] = (unsigned)cdiv(p.n_ctx, 64);
@@ -1117,15 +1172,18 @@ Plan plan_builtin(Kernel &k, const Library &lib, const std::vector<Arg> &args, i
         plan.empty = true;
         return plan;
       }
-      const bool fast = attn_fast_ok(spec, stride_head, stride_seq, n_ctx, sm_scale);
+      const int width = attn_pad_width(spec, heads, stride_head, stride_seq, n_ctx, sm_scale);
+      const bool fast = width || attn_fast_ok(spec, stride_head, stride_seq, n_ctx, sm_scale);
       if (fast) {
         plan.grid[0] = (unsigned)(cdiv(n_ctx, 128) * heads);
       } else {
         plan.grid[0] = (unsigned)cdiv(n_ctx, 64);
         plan.grid[1] = (unsigned)heads;
       }
-      const std::string fast_name = format("tm_attn_%s_fast_%s_d%d%s", dq ? "dq" : "dkdv", el,
-                                           spec.head_dim, spec.causal ? "_causal" : "");
+      const char *op = dq ? "dq" : "dkdv";
+      const std::string fast_name =
+          width ? attn_pad_symbol(op, spec, width)
+                : format("tm_attn_%s_fast_%s_d%d%s", op, el, spec.head_dim, spec.causal ? "_causal" : "");
       plan.block = 256;
       if (dq) {
         TmAttnDqArgs p{};
