@@ -920,7 +920,7 @@ TM_DEV void attn_dq_fast(const TmAttnDqArgs &p, char *lds, int wg, int nwg) {
   }
 }
 
-/* ---- backward: dK, dV ---------------------------------------------------
+/* ---- backward: dK, dV and dQ in one pass (bwd=atomic) -----------------------
  * One workgroup = 4 waves = 128 keys; each wave owns 32 keys, held in
  * registers (K^T and V^T as B operands), and walks the query blocks (BM = 32
  * queries at D = 128, 64 at D = 64) of its head.  Per block, with the lane owning one key:
@@ -939,15 +939,15 @@ TM_DEV void attn_dq_fast(const TmAttnDqArgs &p, char *lds, int wg, int nwg) {
  * are independent, so the wave's VALU work overlaps its MFMA work.  Buffer
  * indices are compile-time (PH = i mod 3) so the compiler sees that the
  * in-flight copy never aliases the tiles being read. */
-template <typename T, int D, bool CAUSAL, bool FUSED = false>
-TM_DEV void attn_dkdv_fast(const TmAttnDkdvArgs &p, float *dq_acc = nullptr) {
+template <typename T, int D, bool CAUSAL>
+TM_DEV void attn_bwd_fused(const TmAttnDkdvArgs &p, float *dq_acc) {
   /* query rows per step: 64 at D = 64 (twice the MFMA work per barrier and
    * per softmax pass; measured 7% faster), 32 at D = 128, where 64 would not
    * fit the registers */
   constexpr int BN = 128, KW = 32, BM = D == 64 ? 64 : 32;
   /* The kernel carries -dS = P (Delta - dP): the dP MFMAs run on -V and start
    * from Delta, so no subtraction per element.  dK accumulates -dK and flips
-   * the sign at the store; FUSED adds dQ with -K. */
+   * the sign at the store; dQ is added with -K. */
   constexpr int QT = BM / 16, KK = BM / 32;
   constexpr int KS = D / 32;
   constexpr int TILE = BM * D * 2;
@@ -956,10 +956,10 @@ TM_DEV void attn_dkdv_fast(const TmAttnDkdvArgs &p, float *dq_acc = nullptr) {
   __shared__ __align__(1024) char lds_0[BUF];
   __shared__ __align__(1024) char lds_1[BUF];
   __shared__ __align__(1024) char lds_2[BUF];
-  /* FUSED: dS of two query blocks, [BN keys][BM queries] each, so that every
+  /* dS of two query blocks, [BN keys][BM queries] each, so that every
    * wave can read all 128 keys of it (ds_off) */
   constexpr int DS_TILE = BN * BM * 2;
-  __shared__ __align__(1024) char lds_ds[FUSED ? 2 * DS_TILE : 16];
+  __shared__ __align__(1024) char lds_ds[2 * DS_TILE];
 
   typedef typename Vec8<T>::type v8;
   const int tid = threadIdx.x, lane = tid & 63;
@@ -1010,14 +1010,14 @@ TM_DEV void attn_dkdv_fast(const TmAttnDkdvArgs &p, float *dq_acc = nullptr) {
       vf[kt][ks] ^= (u32x4){0x80008000u, 0x80008000u, 0x80008000u, 0x80008000u};
     }
   }
-  /* FUSED: K as the B operand of dQ[:, wave's D/4 columns] = dS K, for the
+  /* K as the B operand of dQ[:, wave's D/4 columns] = dS K, for the
    * 128 keys in four 32-key steps; element j of a lane holds key
    * 32 ks + 4g + j (j < 4) or 32 ks + 16 + 4g + j - 4, the order in which the
    * transposing read of dS delivers them.  Keys at or past n are zero, so the
    * (finite) dS of those padding keys adds nothing. */
-  constexpr int NT = FUSED ? D / 64 : 1;
-  u32x4 kq[FUSED ? 4 : 1][NT];
-  if constexpr (FUSED) {
+  constexpr int NT = D / 64;
+  u32x4 kq[4][NT];
+  {
     const uint16_t *Kh = (const uint16_t *)Kg;
 #pragma unroll
     for (int ks = 0; ks < 4; ++ks)
@@ -1119,7 +1119,7 @@ TM_DEV void attn_dkdv_fast(const TmAttnDkdvArgs &p, float *dq_acc = nullptr) {
     }
   };
 
-  /* FUSED: byte offset of queries q .. q+3 (q a multiple of 4) of key row
+  /* byte offset of queries q .. q+3 (q a multiple of 4) of key row
    * `key` in a dS tile; 16-byte chunks XOR-swizzled so that the 16 rows one
    * transposing read spans fall on distinct banks */
   auto ds_off = [&](int key, int q) {
@@ -1190,10 +1190,10 @@ TM_DEV void attn_dkdv_fast(const TmAttnDkdvArgs &p, float *dq_acc = nullptr) {
     u32x4 pf2[2][KK], ds2[2][KK];
     if (!CHECKED || i + 1 < nblocks) {
       scores(edge_tag, nx1, i + 1, pf2, ds2);
-      if constexpr (FUSED) put_ds(i + 1, ds2);
+      put_ds(i + 1, ds2);
     }
     grads(cur, pf, dsf);
-    if constexpr (FUSED) dq_block(i);
+    dq_block(i);
 #pragma unroll
     for (int kt = 0; kt < 2; ++kt)
 #pragma unroll
@@ -1229,10 +1229,8 @@ TM_DEV void attn_dkdv_fast(const TmAttnDkdvArgs &p, float *dq_acc = nullptr) {
   wait_vmem();
   __syncthreads();
   if (nblocks > 0) scores(Edge{}, lds_0, 0, pf, dsf);
-  if constexpr (FUSED) {
-    if (nblocks > 0) put_ds(0, dsf);
-    __syncthreads();
-  }
+  if (nblocks > 0) put_ds(0, dsf);
+  __syncthreads();
 
   /* Block b is masked if it lies in the diagonal band (b < band) or runs past
    * n (b >= full).  Step i masks the softmax of block i+1. */
@@ -1276,30 +1274,37 @@ TM_DEV void attn_dkdv_fast(const TmAttnDkdvArgs &p, float *dq_acc = nullptr) {
 }
 
 
-/* ---- backward: dK, dV at two waves per SIMD -------------------------------
- * The same work split as attn_dkdv_fast (a workgroup of 4 waves owns 128 keys,
- * a wave 32 of them, and walks 32-query blocks), built for two waves per SIMD
- * so that the other workgroup's wave fills the MFMA pipe while this one runs
- * its softmax.  To fit 256 registers the wave keeps only K^T in registers;
- * the workgroup's 128 V rows are copied to LDS once and read per block.
- * Q/dO tiles are double-buffered.  LDS is addressed by 32-bit offsets whose
- * lane parts are computed once (row offsets within a tile are immediates).
- * Scheduling fences sit only between the three phases of a block (score
+/* ---- backward: dK, dV ------------------------------------------------------
+ * The work split of attn_bwd_fused (a workgroup of 4 waves owns 128 keys, a wave
+ * 32 of them) without dQ, built for two waves per SIMD (three at D = 64) so that
+ * the other workgroup's wave fills the MFMA pipe while this one runs its
+ * softmax.  To fit 256 registers the wave keeps only K^T in registers; the
+ * workgroup's 128 V rows are copied to LDS once and read per block.  Q/dO tiles
+ * are double-buffered and contracted 32 queries at a time.  LDS is addressed by
+ * 32-bit offsets whose lane parts are computed once (row offsets within a tile
+ * are immediates).
+ * Scheduling fences sit only between the three phases of 32 queries (score
  * MFMAs, softmax, gradient MFMAs): without them the compiler hoists the whole
  * block's operand reads and spills; finer fences (per k-step or per two d
  * tiles) measured 2-3% slower.  The masked and the interior blocks run in
  * separate loops: a branch between the two forms inside one loop body made
  * the register allocator spill the accumulators.
- * As in attn_dkdv_fast, the dP MFMAs run on -V (negated once in LDS) and
+ * Block rows: 32 at D = 128 (LDS for two workgroups per CU); 64 at D = 64, where
+ * half the barriers pay: f16, 128 heads of 1024 rows 72 us against 77 with 32
+ * rows, one head of 1000 rows 24.4 against 27.1.  One wave per SIMD with K and V
+ * in registers and three buffers took 97 and 24.4 us (128 heads of 4096 causal:
+ * 694 against 522 us).
+ * As in attn_bwd_fused, the dP MFMAs run on -V (negated once in LDS) and
  * start from Delta, so they deliver Delta - dP, and the kernel carries
  * -dS = P (Delta - dP) with one multiply; the arithmetic is the same as that
- * kernel's (and its fused form's), so dK and dV are bit-identical. */
+ * kernel's, so dK and dV are bit-identical. */
 template <int D> struct Dkdv2wLds {
-  static constexpr int BYTES = 128 * D * 2 + 2 * (2 * 32 * D * 2 + 32 * 8);
+  static constexpr int BM = D == 64 ? 64 : 32; /* query rows per copied block */
+  static constexpr int BYTES = 128 * D * 2 + 2 * (2 * BM * D * 2 + BM * 8);
 };
 template <typename T, int D, bool CAUSAL, int DC = D, bool PAD = false>
 TM_DEV void attn_dkdv_2w(const TmAttnDkdvArgs &p, char *lds, int wg, int nwg) {
-  constexpr int BN = 128, KW = 32, BM = 32;
+  constexpr int BN = 128, KW = 32, BM = Dkdv2wLds<D>::BM;
   constexpr int KS = (DC + 31) / 32, DT = DC / 16;
   constexpr int TILE = BM * D * 2;
   constexpr int VT = BN * D * 2;
@@ -1352,9 +1357,9 @@ TM_DEV void attn_dkdv_2w(const TmAttnDkdvArgs &p, char *lds, int wg, int nwg) {
     const int qs = q_start + blk * BM;
     qcp.copy(Qg, ss, qs, n, buf, wave);
     qcp.copy(dOg, ss, qs, n, buf + TILE, wave);
-    if (wave == 0) {
-      const int q = min(qs + (lane & 31), n - 1);
-      lds_copy4_global(lane < 32 ? Lg + q : Dg + q, buf + STATS);
+    if (wave < BM / 32) { /* per 32 queries: L[32] then Delta[32] */
+      const int q = min(qs + wave * 32 + (lane & 31), n - 1);
+      lds_copy4_global(lane < 32 ? Lg + q : Dg + q, buf + STATS + wave * 256);
     }
   };
   vcp.copy(Vg, ss, k0, n, vbase, wave);
@@ -1386,13 +1391,16 @@ TM_DEV void attn_dkdv_2w(const TmAttnDkdvArgs &p, char *lds, int wg, int nwg) {
   for (int dt = 0; dt < DT; ++dt)
     dk[dt][0] = dk[dt][1] = dv[dt][0] = dv[dt][1] = (f32x4){0.f, 0.f, 0.f, 0.f};
 
-  auto block = [&](auto edge_tag, uint32_t cur, int blk) {
+  /* the 32 queries from row 32 * half of block `blk` */
+  auto block = [&](auto edge_tag, auto half_tag, uint32_t cur, int blk) {
     constexpr bool EDGE = decltype(edge_tag)::value;
-    const int qs = q_start + blk * BM;
+    constexpr int HR = decltype(half_tag)::value * 32;             /* rows */
+    constexpr int HB = HR * D * 2, ST = STATS + HR * 8;            /* bytes */
+    const int qs = q_start + blk * BM + HR;
     f32x4 s[2][2], dp[2][2];
 #pragma unroll
     for (int qt = 0; qt < 2; ++qt) {
-      const f32x4 dl = __builtin_bit_cast(f32x4, lds_read16(cur + STATS + 128 + (qt * 16 + 4 * g) * 4));
+      const f32x4 dl = __builtin_bit_cast(f32x4, lds_read16(cur + ST + 128 + (qt * 16 + 4 * g) * 4));
       s[0][qt] = s[1][qt] = (f32x4){0.f, 0.f, 0.f, 0.f};
       dp[0][qt] = dp[1][qt] = dl;
     }
@@ -1400,7 +1408,7 @@ TM_DEV void attn_dkdv_2w(const TmAttnDkdvArgs &p, char *lds, int wg, int nwg) {
     for (int ks = 0; ks < KS; ++ks) {
 #pragma unroll
       for (int qt = 0; qt < 2; ++qt) {
-        const v8 qa = as_vec8<T>(lds_read16(cur + qoff[ks] + qt * 16 * D * 2));
+        const v8 qa = as_vec8<T>(lds_read16(cur + qoff[ks] + HB + qt * 16 * D * 2));
 #pragma unroll
         for (int kt = 0; kt < 2; ++kt) s[kt][qt] = mfma_16x16x32(qa, as_vec8<T>(kf[kt][ks]), s[kt][qt]);
       }
@@ -1409,7 +1417,7 @@ TM_DEV void attn_dkdv_2w(const TmAttnDkdvArgs &p, char *lds, int wg, int nwg) {
         const v8 vb = as_vec8<T>(lds_read16(vbase + voff[ks] + kt * 16 * D * 2));
 #pragma unroll
         for (int qt = 0; qt < 2; ++qt) {
-          const v8 da = as_vec8<T>(lds_read16(cur + TILE + qoff[ks] + qt * 16 * D * 2));
+          const v8 da = as_vec8<T>(lds_read16(cur + TILE + qoff[ks] + HB + qt * 16 * D * 2));
           dp[kt][qt] = mfma_16x16x32(da, vb, dp[kt][qt]);
         }
       }
@@ -1422,7 +1430,7 @@ TM_DEV void attn_dkdv_2w(const TmAttnDkdvArgs &p, char *lds, int wg, int nwg) {
       float pr[2][4], ds[2][4];
 #pragma unroll
       for (int qt = 0; qt < 2; ++qt) {
-        const f32x4 lse = __builtin_bit_cast(f32x4, lds_read16(cur + STATS + (qt * 16 + 4 * g) * 4));
+        const f32x4 lse = __builtin_bit_cast(f32x4, lds_read16(cur + ST + (qt * 16 + 4 * g) * 4));
 #pragma unroll
         for (int r = 0; r < 4; ++r) {
           float x = __builtin_fmaf(s[kt][qt][r], qk_scale, -lse[r]);
@@ -1441,8 +1449,8 @@ TM_DEV void attn_dkdv_2w(const TmAttnDkdvArgs &p, char *lds, int wg, int nwg) {
     }
 #pragma unroll
     for (int dt = 0; dt < DT; ++dt) {
-      const v8 doa = as_vec8<T>(lds_read_kmajor(cur + TILE + kmoff[dt], 0, 16 * D * 2));
-      const v8 qa = as_vec8<T>(lds_read_kmajor(cur + kmoff[dt], 0, 16 * D * 2));
+      const v8 doa = as_vec8<T>(lds_read_kmajor(cur + TILE + kmoff[dt], HB, HB + 16 * D * 2));
+      const v8 qa = as_vec8<T>(lds_read_kmajor(cur + kmoff[dt], HB, HB + 16 * D * 2));
 #pragma unroll
       for (int kt = 0; kt < 2; ++kt) {
         dv[dt][kt] = mfma_16x16x32(doa, as_vec8<T>(pf[kt]), dv[dt][kt]);
@@ -1475,7 +1483,9 @@ TM_DEV void attn_dkdv_2w(const TmAttnDkdvArgs &p, char *lds, int wg, int nwg) {
     /* causal: a block whose every query precedes the wave's first key adds
      * exact zeros; the wave skips its arithmetic (not its copies and barrier),
      * which changes no bit of dK or dV (0.5-1% faster at config 5) */
-    if (!CAUSAL || q_start + (i + 1) * BM > kw0) block(edge_tag, cur, i);
+    static_for<BM / 32>([&](auto h) {
+      if (!CAUSAL || q_start + i * BM + decltype(h)::value * 32 + 32 > kw0) block(edge_tag, h, cur, i);
+    });
     wait_vmem();
     __syncthreads();
   };

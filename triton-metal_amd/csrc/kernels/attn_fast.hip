@@ -16,28 +16,19 @@ TM_PRE_FAST(f16_t, f16, 128)
     __shared__ __align__(1024) char lds[DqLds<D>::BYTES];                                     \
     attn_dq_fast<T, D, CAUSAL>(p, lds, blockIdx.x, gridDim.x);                                \
   }                                                                                           \
-  TM_DKDV_FAST_##D(T, TN, CAUSAL, CN)
-/* head_dim 128: the two-waves-per-SIMD kernel (0.99-1.03 ms at B4 H32 S4096
- * causal against 1.11-1.16 ms for attn_dkdv_fast at one wave per SIMD, whose
- * dK, dV accumulators plus K^T and V^T fragments need more than 256
- * registers); head_dim 64: attn_dkdv_fast, one wave per SIMD */
-#define TM_DKDV_FAST_128(T, TN, CAUSAL, CN)                                                   \
+  TM_DKDV_FAST(T, TN, D, CAUSAL, CN)
+#define TM_DKDV_FAST(T, TN, D, CAUSAL, CN)                                                    \
   extern "C" __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void  \
-  tm_attn_dkdv_fast_##TN##_d128##CN(TmAttnDkdvArgs p) {                                       \
-    __shared__ __align__(1024) char lds[Dkdv2wLds<128>::BYTES];                                    \
-    attn_dkdv_2w<T, 128, CAUSAL>(p, lds, blockIdx.x, gridDim.x);                              \
-  }
-#define TM_DKDV_FAST_64(T, TN, CAUSAL, CN)                                                    \
-  extern "C" __global__ __launch_bounds__(256) void tm_attn_dkdv_fast_##TN##_d64##CN(         \
-      TmAttnDkdvArgs p) {                                                                     \
-    attn_dkdv_fast<T, 64, CAUSAL>(p);                                                         \
+  tm_attn_dkdv_fast_##TN##_d##D##CN(TmAttnDkdvArgs p) {                                       \
+    __shared__ __align__(1024) char lds[Dkdv2wLds<D>::BYTES];                                 \
+    attn_dkdv_2w<T, D, CAUSAL>(p, lds, blockIdx.x, gridDim.x);                                \
   }
 /* Single-pass backward with atomic dQ (opt-in: bwd=atomic): the dK/dV
  * kernel plus dQ = dS K per query block, and the passes around it. */
 #define TM_BWD_FUSED(T, TN, D, CAUSAL, CN)                                                    \
   extern "C" __global__ __launch_bounds__(256) void tm_attn_fused_fast_##TN##_d##D##CN(       \
       TmAttnFusedArgs p) {                                                                    \
-    attn_dkdv_fast<T, D, CAUSAL, true>(p.kv, p.dq_acc);                                       \
+    attn_bwd_fused<T, D, CAUSAL>(p.kv, p.dq_acc);                                       \
   }
 #define TM_BWD_FAST_ALL(T, TN)           \
   TM_BWD_FUSED(T, TN, 64, false, )       \
