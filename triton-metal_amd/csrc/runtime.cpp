@@ -673,17 +673,19 @@ bool gemm_w4_enabled() {
 
 /* Kernel choice shared by matmul_kernel and sae_encode_kernel.  The
  * specialised kernels take 16-bit elements and row-major operands with unit
- * inner stride, 16-byte aligned rows of A and B, 8-byte aligned rows of C,
- * and rows no shorter than the matrix (lda >= K, ldb >= N): whole tiles (and
- * K a multiple of 64) run the aligned kernel, any other M, N, K the ragged
- * one, whose copies clip at the matrix's last row and whose last k-step and
- * stores are masked.  Either operand (not both) may instead be stored
+ * inner stride, 16-byte aligned rows of A and B
+ * and rows no shorter than the matrix (lda >= K, ldb >= N): whole tiles (K a
+ * multiple of 64, 8-byte aligned rows of C) run the aligned kernel, any other
+ * M, N, K the ragged one, whose copies clip at the matrix's last row and whose
+ * last k-step and stores are masked.  Rows of A or B at other addresses run the
+ * unaligned kernels, whose tiles go through registers (2049 x 4097 x 1025 bf16:
+ * 50 us against 454 on the generic fp32-MFMA kernel).  Either operand (not both) may instead be stored
  * transposed: B with unit stride along K (the x @ W^T layout), read like A,
  * or A with unit stride along M (dY^T X), read like B.  fp32 with the same
  * layouts, 16-byte aligned rows and whole 128 x 128 (or, for problems with
  * few of those, 64 x 64) x 32 tiles runs the fp32 MFMA kernel.  Anything else
  * runs the generic 64 x 64 kernel. */
-void choose_gemm(Plan &plan, const TmGemmArgs &p, const BuiltinSpec &spec, const char *family) {
+void choose_gemm(Plan &plan, TmGemmArgs &p, const BuiltinSpec &spec, const char *family) {
   const char *el = element_name(spec.element);
   /* fp32: whole 128 x 128 x 32 tiles on the fp32 MFMA kernel when there are
    * at least half as many of them as compute units, else whole 64 x 64 tiles
@@ -717,19 +719,30 @@ void choose_gemm(Plan &plan, const TmGemmArgs &p, const BuiltinSpec &spec, const
       return;
     }
   }
-  const bool half = fast_paths_enabled() && spec.element != Element::F32 && p.scn == 1 &&
-                    p.k > 0 && p.scm % 4 == 0;
+  const bool half = fast_paths_enabled() && spec.element != Element::F32 && p.scn == 1 && p.k > 0;
   /* A row-major [M, K], or (matmul only) stored transposed: element (m, k) at
    * k * stride_ak + m, the dY^T X layout */
-  const bool a_n = half && p.sak == 1 && p.sam % 8 == 0 && p.sam >= p.k && p.sam <= (1 << 26);
-  const bool a_t = half && !a_n && gemm && p.sam == 1 && p.sak % 8 == 0 && p.sak >= p.m &&
+  const bool a_n = half && p.sak == 1 && p.sam >= p.k && p.sam <= (1 << 26);
+  const bool a_t = half && !(a_n && p.sam % 8 == 0) && gemm && p.sam == 1 && p.sak >= p.m &&
                    p.sak <= (1 << 26);
   /* B row-major [K, N], or (matmul only) stored transposed: element (k, n) at
    * n * stride_bn + k, the x @ W^T layout */
-  const bool b_n = p.sbn == 1 && p.sbk % 8 == 0 && p.sbk >= p.n && p.sbk <= (1 << 26);
-  const bool b_t = !b_n && gemm && p.sbk == 1 && p.sbn % 8 == 0 && p.sbn >= p.k && p.sbn <= (1 << 26);
-  const bool nn = a_n && b_n, nt = a_n && b_t, tn = a_t && b_n;
+  const bool b_n = p.sbn == 1 && p.sbk >= p.n && p.sbk <= (1 << 26);
+  const bool b_t = !(b_n && p.sbk % 8 == 0) && gemm && p.sbk == 1 && p.sbn >= p.k && p.sbn <= (1 << 26);
+  /* rows of an operand that start 16-byte aligned; where both strides are 1 the
+   * aligned reading wins, as a matrix of one row or column has two */
+  const bool a_t8 = a_t && p.sak % 8 == 0, b_t8 = b_t && p.sbn % 8 == 0;
+  const bool a_n8 = a_n && p.sam % 8 == 0, b_n8 = b_n && p.sbk % 8 == 0;
+  const bool aligned = (a_n8 && (b_n8 || b_t8)) || (a_t8 && b_n8);
+  /* unaligned tiles are addressed by 32-bit byte offsets over up to 256 rows */
+  const int32_t ld_limit = 1 << 22;
+  const bool fits = (p.sak == 1 ? p.sam : p.sak) < ld_limit && (p.sbn == 1 ? p.sbk : p.sbn) < ld_limit;
+  const bool nn = aligned ? a_n8 && b_n8 : fits && a_n && b_n;
+  const bool nt = !nn && (aligned ? a_n8 && b_t8 : fits && a_n && b_t);
+  const bool tn = !nn && !nt && (aligned ? a_t8 && b_n8 : fits && a_t && b_n);
+  p.layout = TM_GEMM_ANY;
   if (nn || nt || tn) {
+    p.layout = nn ? TM_GEMM_NN : nt ? TM_GEMM_NT : TM_GEMM_TN;
     /* 256 x 256 tiles (512 threads, one resident per compute unit) or 128 x
      * 128 tiles (256 threads, two resident), whichever needs less time by
      * rounds of resident tiles: a round of 256 x 256 tiles takes about 31/21
@@ -738,12 +751,15 @@ void choose_gemm(Plan &plan, const TmGemmArgs &p, const BuiltinSpec &spec, const
      * 650 on 256 x 256) */
     const int64_t cus = std::max(device().compute_units, 1);
     const bool big = cdiv(cdiv(p.m, 256) * cdiv(p.n, 256), cus) * 31 <=
-                     cdiv(cdiv(p.m, 128) * cdiv(p.n, 128), 2 * cus) * 21;
+                         cdiv(cdiv(p.m, 128) * cdiv(p.n, 128), 2 * cus) * 21 &&
+                     /* (the 256 x 256 unaligned kernel would spill with A transposed) */
+                     (aligned || !tn);
     /* with fewer 128 x 128 tiles than compute units, 64 x 64 tiles (128
      * threads): 1024^3 bf16 had 64 tiles of 128 x 128 */
     const bool small = !big && cdiv(p.m, 128) * cdiv(p.n, 128) < cus;
     const int tile = big ? 256 : small ? 64 : 128;
-    const bool whole = p.m % tile == 0 && p.n % tile == 0 && p.k % 64 == 0;
+    const bool whole =
+        aligned && p.m % tile == 0 && p.n % tile == 0 && p.k % 64 == 0 && p.scm % 4 == 0;
     const int64_t tiles = cdiv(p.m, tile) * cdiv(p.n, tile);
     /* whole row-major tiles with fewer 128 x 128 workgroups than two per CU
      * (one wave per SIMD), or 64 x 64 ones (two waves each): the K loop split
@@ -753,8 +769,8 @@ void choose_gemm(Plan &plan, const TmGemmArgs &p, const BuiltinSpec &spec, const
     const bool ksplit = TM_GEMM_KSPLIT && gemm && nn && whole && !big && p.k >= 128 &&
                         (small ? tiles <= 2 * cus : tiles < 2 * cus);
     const int kg = !ksplit ? 1 : small && tiles > cus ? 2 : small ? 4 : 2;
-    plan.variant = format("tm_%s_%s%s%s%s_%s", family, whole ? "fast" : "ragged",
-                          nt ? "_nt" : tn ? "_tn" : "", big ? "" : small ? "_t64" : "_t128",
+    plan.variant = format("tm_%s_%s%s%s%s_%s", family,
+                          whole ? "fast" : aligned ? "ragged" : "unaligned", nt ? "_nt" : tn ? "_tn" : "", big ? "" : small ? "_t64" : "_t128",
                           kg == 4 ? "_k4" : kg == 2 ? "_k2" : "", el);
     plan.grid[0] = (unsigned)tiles;
     plan.block = (unsigned)(2 * tile * kg);
@@ -764,6 +780,8 @@ void choose_gemm(Plan &plan, const TmGemmArgs &p, const BuiltinSpec &spec, const
      * 64 of the other kind */
     const int64_t a_rows = a_n ? (int64_t)p.sam * 512 : (int64_t)p.sak * 128;
     const int64_t b_rows = b_t ? (int64_t)p.sbn * 512 : (int64_t)p.sbk * 128;
+    /* 64 x 64 unaligned tiles: the generic kernels, all layouts in one */
+    if (!aligned && small) plan.variant = format("tm_%s_generic_%s", family, el);
     if (gemm_w4_enabled() && whole && big && a_rows <= INT32_MAX && b_rows <= INT32_MAX) {
       plan.variant = format("tm_%s_w4%s_%s", family, nt ? "_nt" : tn ? "_tn" : "", el);
       plan.block = 256;
@@ -867,8 +885,10 @@ bool plan_gemm_split(Plan &plan, TmGemmArgs &p, const BuiltinSpec &spec, const L
                      const Scratch *scratch) {
   /* the split is compiled into "_ks" instantiations of the 64 x 64-tile
    * GEMM kernels only */
-  if (!TM_GEMM_SPLITK || spec.element == Element::F32 || plan.variant.find("_t64") == std::string::npos ||
-      plan.variant.rfind("tm_gemm_", 0) != 0)
+  const char *el = element_name(spec.element);
+  const bool unaligned = p.layout != TM_GEMM_ANY && plan.variant == format("tm_gemm_generic_%s", el);
+  if (!TM_GEMM_SPLITK || spec.element == Element::F32 || plan.variant.rfind("tm_gemm_", 0) != 0 ||
+      (!unaligned && plan.variant.find("_t64") == std::string::npos))
     return false;
   const int64_t cus = std::max(device().compute_units, 1);
   const int64_t tiles = plan.grid[0];
@@ -884,11 +904,13 @@ bool plan_gemm_split(Plan &plan, TmGemmArgs &p, const BuiltinSpec &spec, const L
   p.splits = (int32_t)splits;
   Plan main = plan, reduce;
   /* the "_ks" instantiation of the planned kernel */
-  const std::string suffix = std::string("_") + element_name(spec.element);
-  main.variant = plan.variant.substr(0, plan.variant.size() - suffix.size()) + "_ks" + suffix;
+  const std::string suffix = std::string("_") + el;
+  main.variant = unaligned ? format("tm_gemm_unaligned%s_t64_ks_%s",
+                                    p.layout == TM_GEMM_NT ? "_nt" : p.layout == TM_GEMM_TN ? "_tn" : "", el)
+                           : plan.variant.substr(0, plan.variant.size() - suffix.size()) + "_ks" + suffix;
   main.grid[1] = (unsigned)splits;
   set_kernarg(main, p);
-  reduce.variant = format("tm_gemm_split_reduce_%s", element_name(spec.element));
+  reduce.variant = format("tm_gemm_split_reduce_%s", el);
   reduce.grid[0] = (unsigned)cdiv((int64_t)p.m * (np / 4), 256);
   reduce.block = 256;
   set_kernarg(reduce, p);
@@ -1822,12 +1844,12 @@ int64_t tm_alloc_buffer(int64_t length) {
     throw TmError(format("buffer length must be positive, got %lld", (long long)length));
   require_device();
   auto buf = std::make_shared<Buffer>();
-  /* Padded to 256 bytes: the GEMM's 16-byte tile copies may read up to 14
-   * bytes past the end of a matrix whose rows are not a multiple of 8
-   * elements (those bytes feed only outputs that are not stored). */
-  if (length > INT64_MAX - 255)
+  /* 16 bytes more than asked for, to whole 256 bytes: the GEMM's 16-byte tile
+   * loads may read up to 14 bytes past the end of a matrix whose rows are not a
+   * multiple of 8 elements (those bytes feed only outputs that are not stored). */
+  if (length > INT64_MAX - 271)
     throw TmError(format("could not allocate a %lld-byte device buffer (too large)", (long long)length));
-  hipError_t status = hipMalloc(&buf->ptr, (size_t)((length + 255) & ~(int64_t)255));
+  hipError_t status = hipMalloc(&buf->ptr, (size_t)((length + 16 + 255) & ~(int64_t)255));
   if (status != hipSuccess) {
     buf->ptr = nullptr;
     (void)hipGetLastError();

@@ -18,6 +18,10 @@
 
 #include <stdint.h>
 
+/* which strides of A and B are 1: any, both inner ones (row-major), B's along K
+ * (B stored transposed), A's along M (A stored transposed) */
+enum TmGemmLayout { TM_GEMM_ANY = 0, TM_GEMM_NN = 1, TM_GEMM_NT = 2, TM_GEMM_TN = 3 };
+
 struct TmGemmArgs {
   const void *a;
   const void *b;
@@ -29,6 +33,7 @@ struct TmGemmArgs {
    * [splits][m][round4(n)], summed into c by the reduce dispatch */
   float *part;
   int32_t splits;
+  int32_t layout; /* TmGemmLayout; read by the 16-bit generic kernels */
 };
 
 struct TmAttnFwdArgs {
