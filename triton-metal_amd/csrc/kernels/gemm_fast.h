@@ -272,7 +272,7 @@ TM_DEV uint32_t g_pack2(float lo, float hi) {
  * dY^T X in a linear layer's weight gradient).  Its tile is then [64 x BM]
  * m-contiguous like B's, copied and read the same way (transposed reads). */
 /* KG: groups of 2 WN waves splitting the K loop inside the workgroup (1, 2
- * or 4; whole tiles only).  Group h contracts k-steps h, h + KG, ... from its
+ * or 4).  Group h contracts k-steps h, h + KG, ... from its
  * own double-buffered tiles; at the end groups 1 .. KG-1 leave their
  * accumulators in LDS and group 0 adds them in order and stores.  For grids
  * of about one workgroup per CU (128 x 128 tiles at 2048^3, 64 x 64 at
@@ -280,12 +280,23 @@ TM_DEV uint32_t g_pack2(float lo, float hi) {
 /* KSPLIT: the K range of the workgroup comes from grid y and p.splits, and
  * the result is an fp32 partial (64 x 64 tiles only: the instantiations the
  * planner uses when the tiles alone leave the chip idle). */
-/* UNAL: rows of A and B at any address; the tiles' LDS is the caller's (a kernel
- * of several instantiations shares it). */
-constexpr int unaligned_lds(int tile) { return 2 * 2 * tile * GBK * 2; }
+/* The LDS of a kernel's tiles: those of K group 0 (four arrays, which the
+ * compiler then knows do not alias, or parts of one) and group_lds(tile) bytes
+ * for each further group. */
+constexpr int group_lds(int tile) { return 2 * 2 * tile * GBK * 2; }
+template <bool ONE> /* all in one array, group after group */
+struct GemmTiles {
+  char *a0, *b0, *a1, *b1, *more;
+};
+template <int TILE>
+TM_DEV GemmTiles<true> tiles_at(char *lds) {
+  constexpr int HALF = TILE * GBK * 2;
+  return {lds, lds + HALF, lds + 2 * HALF, lds + 3 * HALF, lds + group_lds(TILE)};
+}
+/* UNAL: rows of A and B at any address. */
 template <typename T, int EPI, bool RAGGED, int BM, int BN, bool BT = false, bool AT = false,
-          int KG = 1, bool KSPLIT = false, bool UNAL = false>
-TM_DEV void gemm_fast(const TmGemmArgs &p, char *unal_lds = nullptr) {
+          int KG = 1, bool KSPLIT = false, bool UNAL = false, bool ONE>
+TM_DEV void gemm_fast(const TmGemmArgs &p, const GemmTiles<ONE> tiles) {
   static_assert(!UNAL || RAGGED, "unaligned rows: any M, N, K");
   typedef typename GVec8<T>::type v8;
   constexpr int GBM = BM, GBN = BN;
@@ -296,18 +307,20 @@ TM_DEV void gemm_fast(const TmGemmArgs &p, char *unal_lds = nullptr) {
   static_assert((BM == 256 && BN == 256) || (BM == 128 && BN == 128) || (BM == 64 && BN == 64),
                 "tile shapes");
   constexpr int GROUP_BYTES = 2 * (A_TILE + B_TILE);
-  static_assert(KG == 1 || (!RAGGED && GROUP_BYTES >= 2 * WN * MI * 4 * 64 * 16),
-                "K groups: whole tiles, and a group's tiles hold its accumulators");
+  static_assert(KG == 1 || GROUP_BYTES >= 2 * WN * MI * 4 * 64 * 16,
+                "K groups: a group's tiles hold its accumulators");
   const int tid = threadIdx.x, lane = tid & 63;
-  const int kgrp = KG == 1 ? 0 : (tid >> 6) / (2 * WN); /* K group */
-  /* the kernel body over its LDS: one workgroup-wide group takes four
-   * separate tile arrays (the compiler then knows they do not alias), K
-   * groups one array carved per group (`lds`, also where the groups'
-   * accumulators meet) */
-  auto body = [&](char *const lds_a0, char *const lds_b0, char *const lds_a1, char *const lds_b1,
-                  char *const lds) __attribute__((always_inline)) {
+  /* K group, uniform: a wave's branches on its k-step hold barriers */
+  const int kgrp = KG == 1 ? 0 : __builtin_amdgcn_readfirstlane(tid >> 6) / (2 * WN);
+  char *const mine = ONE ? tiles.a0 + kgrp * GROUP_BYTES : tiles.more + (kgrp - 1) * GROUP_BYTES;
+  const bool first = KG == 1 || (!ONE && kgrp == 0);
+  char *const lds_a0 = first ? tiles.a0 : mine;
+  char *const lds_b0 = first ? tiles.b0 : mine + A_TILE;
+  char *const lds_a1 = first ? tiles.a1 : mine + A_TILE + B_TILE;
+  char *const lds_b1 = first ? tiles.b1 : mine + 2 * A_TILE + B_TILE;
   /* uniform in the ragged kernel, whose copy ranges are scalar arithmetic */
-  const int wave = RAGGED ? __builtin_amdgcn_readfirstlane(tid >> 6) : KG == 1 ? tid >> 6 : (tid >> 6) % (2 * WN);
+  const int wave_all = RAGGED ? __builtin_amdgcn_readfirstlane(tid >> 6) : tid >> 6;
+  const int wave = KG == 1 ? wave_all : wave_all % (2 * WN);
   const int g = lane >> 4, c = lane & 15;
   const int wm = wave / WN, wn = wave % WN; /* 2 x WN waves */
 
@@ -382,10 +395,10 @@ TM_DEV void gemm_fast(const TmGemmArgs &p, char *unal_lds = nullptr) {
   if constexpr (UNAL) {
     ua.init(lda, a_rows, a_rows, wave, lane);
     ub.init(ldb, b_cols, b_cols, wave, lane);
-    if (kbeg < kend) {
-      load_ua(kbeg);
+    if (kbeg + kgrp < kend) {
+      load_ua(kbeg + kgrp);
       ua.store(lds_a0);
-      load_ub(kbeg);
+      load_ub(kbeg + kgrp);
       ub.store(lds_b0);
     }
   } else {
@@ -400,9 +413,9 @@ TM_DEV void gemm_fast(const TmGemmArgs &p, char *unal_lds = nullptr) {
   auto step = [&](auto last_tag, const char *ca, const char *cb, char *na, char *nb, int kb) {
     constexpr bool LAST = decltype(last_tag)::value;
     if constexpr (UNAL) {
-      if (!LAST && kb + 1 < kend) {
-        load_ua(kb + 1);
-        if (!IN_TURN) load_ub(kb + 1);
+      if (!LAST && kb + KG < kend) {
+        load_ua(kb + KG);
+        if (!IN_TURN) load_ub(kb + KG);
       }
       __builtin_amdgcn_sched_barrier(0); /* the loads first, behind the MFMAs */
     } else {
@@ -441,20 +454,20 @@ TM_DEV void gemm_fast(const TmGemmArgs &p, char *unal_lds = nullptr) {
       if (LAST) __builtin_amdgcn_sched_barrier(0);
       if (UNAL && IN_TURN && ks == 0) {
         __builtin_amdgcn_sched_barrier(0);
-        if (!LAST && kb + 1 < kend) {
+        if (!LAST && kb + KG < kend) {
           ua.store(na);
-          load_ub(kb + 1);
+          load_ub(kb + KG);
         }
         __builtin_amdgcn_sched_barrier(0);
       }
     }
     if constexpr (UNAL) {
-      if (!LAST && kb + 1 < kend) {
+      if (!LAST && kb + KG < kend) {
         if (!IN_TURN) ua.store(na);
         ub.store(nb);
       }
     }
-    if (!LAST) {
+    if (!LAST || KG != 1) {
       if (!UNAL) g_wait_vmem();
       __syncthreads();
     }
@@ -475,14 +488,20 @@ TM_DEV void gemm_fast(const TmGemmArgs &p, char *unal_lds = nullptr) {
     }
   } else {
     const int rounds = (kend - kbeg + KG - 1) / KG;
+    /* the group whose turn the ragged last step is runs it masked, beside the
+     * others' whole steps: each meets one barrier a round */
+    auto turn = [&](char *ca, char *cb, char *na, char *nb, int kb) {
+      if (RAGGED && kb == kfull && kfull < kend) step(Last{}, ca, cb, na, nb, kb);
+      else step(Full{}, ca, cb, na, nb, kb);
+    };
     for (int r = 0; r < rounds; r += 2) {
-      step(Full{}, lds_a0, lds_b0, lds_a1, lds_b1, kbeg + r * KG + kgrp);
-      if (r + 1 < rounds) step(Full{}, lds_a1, lds_b1, lds_a0, lds_b0, kbeg + (r + 1) * KG + kgrp);
+      turn(lds_a0, lds_b0, lds_a1, lds_b1, kbeg + r * KG + kgrp);
+      if (r + 1 < rounds) turn(lds_a1, lds_b1, lds_a0, lds_b0, kbeg + (r + 1) * KG + kgrp);
     }
     /* groups 1 .. KG-1 leave their partial C^T tiles in their own LDS (the
      * last barrier above ended every read of it); group 0 adds them */
     auto slot = [&](int grp, int i, int j) {
-      return (f32x4 *)(lds + grp * GROUP_BYTES) + (((wave * MI + i) * 4 + j) * 64 + lane);
+      return (f32x4 *)(tiles.more + (grp - 1) * GROUP_BYTES) + (((wave * MI + i) * 4 + j) * 64 + lane);
     };
     if (kgrp > 0) {
 #pragma unroll
@@ -554,19 +573,20 @@ TM_DEV void gemm_fast(const TmGemmArgs &p, char *unal_lds = nullptr) {
       }
     }
   }
-  };
-  if constexpr (UNAL) {
-    body(unal_lds, unal_lds + A_TILE, unal_lds + A_TILE + B_TILE, unal_lds + 2 * A_TILE + B_TILE, nullptr);
-  } else if constexpr (KG == 1) {
-    __shared__ __align__(1024) char tile_a0[A_TILE];
-    __shared__ __align__(1024) char tile_b0[B_TILE];
-    __shared__ __align__(1024) char tile_a1[A_TILE];
-    __shared__ __align__(1024) char tile_b1[B_TILE];
-    body(tile_a0, tile_b0, tile_a1, tile_b1, nullptr);
-  } else {
-    __shared__ __align__(1024) char lds[KG * GROUP_BYTES];
-    char *const mine = lds + kgrp * GROUP_BYTES;
-    body(mine, mine + A_TILE, mine + A_TILE + B_TILE, mine + 2 * A_TILE + B_TILE, lds);
+}
+
+/* As many K groups as the launch has waves for: 1, 2 or 4 of 64 x 64 tiles (128
+ * threads each), 1 or 2 of 128 x 128 (256).  One body each: with the count a
+ * variable, one group of a ragged 1400 x 1400 x 136 ran 7.3 us against 6.4; beside
+ * the other bodies it still runs 6.6, so many tiles, which take one group, have
+ * kernels of their own ("_g1"). */
+template <typename T, int EPI, bool RAGGED, int TILE, bool BT, bool AT, bool UNAL, bool ONE>
+TM_DEV void gemm_groups(const TmGemmArgs &p, const GemmTiles<ONE> tiles) {
+  switch (blockDim.x / (2 * TILE)) {
+    case 1: gemm_fast<T, EPI, RAGGED, TILE, TILE, BT, AT, 1, false, UNAL>(p, tiles); break;
+    case 2: gemm_fast<T, EPI, RAGGED, TILE, TILE, BT, AT, 2, false, UNAL>(p, tiles); break;
+    default:
+      if constexpr (TILE == 64) gemm_fast<T, EPI, RAGGED, TILE, TILE, BT, AT, 4, false, UNAL>(p, tiles);
   }
 }
 

@@ -15,37 +15,46 @@
 #include "gemm_fast.h"
 #include "gemm_generic.h"
 
-static_assert((GENERIC_A + GENERIC_B) * 4 <= unaligned_lds(64), "shared LDS");
+static_assert((GENERIC_A + GENERIC_B) * 4 <= TM_GEMM_GROUP_LDS && group_lds(64) == TM_GEMM_GROUP_LDS, "shared LDS");
 
-#define TM_GEMM_UNAL(NAME, T, EPI, TILE, BT, AT, KS)                                          \
+#define TM_GEMM_UNAL(NAME, T, EPI, TILE, BT, AT)                                              \
   extern "C" __global__ __launch_bounds__(TILE * 2) void NAME(TmGemmArgs p) {                 \
-    __shared__ __align__(1024) char lds[unaligned_lds(TILE)];                                 \
-    gemm_fast<T, EPI, true, TILE, TILE, BT, AT, 1, KS, true>(p, lds);                         \
+    __shared__ __align__(1024) char lds[group_lds(TILE)];                                     \
+    gemm_fast<T, EPI, true, TILE, TILE, BT, AT, 1, false, true>(p, tiles_at<TILE>(lds));                      \
   }
-#define TM_GEMM_UNAL_TILE(T, TN, SUFFIX, TILE)                                                \
-  TM_GEMM_UNAL(tm_gemm_unaligned##SUFFIX##_##TN, T, EPI_NONE, TILE, false, false, false)      \
-  TM_GEMM_UNAL(tm_gemm_unaligned_nt##SUFFIX##_##TN, T, EPI_NONE, TILE, true, false, false)    \
-  TM_GEMM_UNAL(tm_sae_unaligned##SUFFIX##_##TN, T, EPI_BIAS_RELU, TILE, false, false, false)
+/* 64 x 64 tiles with K ranges across workgroups */
+#define TM_GEMM_UNAL_KS(NAME, T, BT, AT, KG)                                                  \
+  extern "C" __global__ __launch_bounds__(128 * KG) void NAME(TmGemmArgs p) {                 \
+    __shared__ __align__(1024) char lds[KG * group_lds(64)];                                  \
+    gemm_fast<T, EPI_NONE, true, 64, 64, BT, AT, KG, true, true>(p, tiles_at<64>(lds));       \
+  }
 #define TM_GEMM_UNAL_ALL(T, TN)                                                               \
-  TM_GEMM_UNAL_TILE(T, TN, , 256)                                                             \
-  TM_GEMM_UNAL_TILE(T, TN, _t128, 128)                                                        \
-  TM_GEMM_UNAL(tm_gemm_unaligned_tn_t128_##TN, T, EPI_NONE, 128, false, true, false)          \
-  TM_GEMM_UNAL(tm_gemm_unaligned_t64_ks_##TN, T, EPI_NONE, 64, false, false, true)            \
-  TM_GEMM_UNAL(tm_gemm_unaligned_nt_t64_ks_##TN, T, EPI_NONE, 64, true, false, true)          \
-  TM_GEMM_UNAL(tm_gemm_unaligned_tn_t64_ks_##TN, T, EPI_NONE, 64, false, true, true)          \
-  extern "C" __global__ __launch_bounds__(256) void tm_gemm_generic_##TN(TmGemmArgs p) {      \
-    __shared__ __align__(1024) char lds[unaligned_lds(64)];                                   \
+  TM_GEMM_UNAL(tm_gemm_unaligned_##TN, T, EPI_NONE, 256, false, false)                       \
+  TM_GEMM_UNAL(tm_gemm_unaligned_nt_##TN, T, EPI_NONE, 256, true, false)                     \
+  TM_GEMM_UNAL(tm_sae_unaligned_##TN, T, EPI_BIAS_RELU, 256, false, false)                   \
+  TM_GEMM_UNAL(tm_gemm_unaligned_t128_##TN, T, EPI_NONE, 128, false, false)                  \
+  TM_GEMM_UNAL(tm_gemm_unaligned_nt_t128_##TN, T, EPI_NONE, 128, true, false)                \
+  TM_GEMM_UNAL(tm_gemm_unaligned_tn_t128_##TN, T, EPI_NONE, 128, false, true)                \
+  TM_GEMM_UNAL(tm_sae_unaligned_t128_##TN, T, EPI_BIAS_RELU, 128, false, false)              \
+  TM_GEMM_UNAL_KS(tm_gemm_unaligned_t64_ks_##TN, T, false, false, 1)                          \
+  TM_GEMM_UNAL_KS(tm_gemm_unaligned_t64_k4_ks_##TN, T, false, false, 4)                       \
+  TM_GEMM_UNAL_KS(tm_gemm_unaligned_nt_t64_ks_##TN, T, true, false, 1)                        \
+  TM_GEMM_UNAL_KS(tm_gemm_unaligned_nt_t64_k4_ks_##TN, T, true, false, 4)                     \
+  TM_GEMM_UNAL_KS(tm_gemm_unaligned_tn_t64_ks_##TN, T, false, true, 1)                        \
+  TM_GEMM_UNAL_KS(tm_gemm_unaligned_tn_t64_k4_ks_##TN, T, false, true, 4)                     \
+  extern "C" __global__ __launch_bounds__(512) void tm_gemm_generic_##TN(TmGemmArgs p) {      \
+    extern __shared__ __align__(1024) char lds[];                                             \
     switch (p.layout) {                                                                       \
-      case TM_GEMM_NN: gemm_fast<T, EPI_NONE, true, 64, 64, false, false, 1, false, true>(p, lds); break; \
-      case TM_GEMM_NT: gemm_fast<T, EPI_NONE, true, 64, 64, true, false, 1, false, true>(p, lds); break;  \
-      case TM_GEMM_TN: gemm_fast<T, EPI_NONE, true, 64, 64, false, true, 1, false, true>(p, lds); break;  \
-      default: gemm_generic<T, EPI_NONE>(p, (float *)lds, (float *)lds + GENERIC_A);                                                \
+      case TM_GEMM_NN: gemm_groups<T, EPI_NONE, true, 64, false, false, true>(p, tiles_at<64>(lds)); break; \
+      case TM_GEMM_NT: gemm_groups<T, EPI_NONE, true, 64, true, false, true>(p, tiles_at<64>(lds)); break;  \
+      case TM_GEMM_TN: gemm_groups<T, EPI_NONE, true, 64, false, true, true>(p, tiles_at<64>(lds)); break;  \
+      default: gemm_generic<T, EPI_NONE>(p, (float *)lds, (float *)lds + GENERIC_A);          \
     }                                                                                         \
   }                                                                                           \
-  extern "C" __global__ __launch_bounds__(256) void tm_sae_generic_##TN(TmGemmArgs p) {       \
-    __shared__ __align__(1024) char lds[unaligned_lds(64)];                                   \
-    if (p.layout == TM_GEMM_NN) gemm_fast<T, EPI_BIAS_RELU, true, 64, 64, false, false, 1, false, true>(p, lds); \
-    else gemm_generic<T, EPI_BIAS_RELU>(p, (float *)lds, (float *)lds + GENERIC_A);                                                   \
+  extern "C" __global__ __launch_bounds__(512) void tm_sae_generic_##TN(TmGemmArgs p) {       \
+    extern __shared__ __align__(1024) char lds[];                                             \
+    if (p.layout == TM_GEMM_NN) gemm_groups<T, EPI_BIAS_RELU, true, 64, false, false, true>(p, tiles_at<64>(lds)); \
+    else gemm_generic<T, EPI_BIAS_RELU>(p, (float *)lds, (float *)lds + GENERIC_A);           \
   }
 TM_GEMM_UNAL_ALL(bf16_t, bf16)
 TM_GEMM_UNAL_ALL(f16_t, f16)

@@ -514,6 +514,7 @@ struct Plan {
   std::string variant;
   unsigned grid[3] = {1, 1, 1};
   unsigned block = 0; /* must be set by the planner; 0 is refused at enqueue */
+  unsigned lds = 0;   /* bytes of LDS beside the kernel's own */
   std::vector<unsigned char> kernarg; /* packed bytes */
   bool empty = false;                 /* nothing to compute (a zero-sized problem) */
   bool by_value_struct = true;        /* built-in: one struct argument */
@@ -761,19 +762,40 @@ void choose_gemm(Plan &plan, TmGemmArgs &p, const BuiltinSpec &spec, const char 
     const bool whole =
         aligned && p.m % tile == 0 && p.n % tile == 0 && p.k % 64 == 0 && p.scm % 4 == 0;
     const int64_t tiles = cdiv(p.m, tile) * cdiv(p.n, tile);
-    /* whole row-major tiles with fewer 128 x 128 workgroups than two per CU
-     * (one wave per SIMD), or 64 x 64 ones (two waves each): the K loop split
-     * over wave groups inside the workgroup -- 128 x 128 tiles over 2 (512
-     * threads); 64 x 64 tiles over 4 (512 threads, one workgroup per CU) up to
-     * one tile per CU, else over 2 (256 threads, two per CU) up to two */
-    const bool ksplit = TM_GEMM_KSPLIT && gemm && nn && whole && !big && p.k >= 128 &&
-                        (small ? tiles <= 2 * cus : tiles < 2 * cus);
+    /* fewer 128 x 128 workgroups than two per CU (one wave per SIMD), or 64 x
+     * 64 ones (two waves each): the K loop split over wave groups inside the
+     * workgroup -- whole 128 x 128 tiles over 2 (512 threads); 64 x 64 tiles
+     * over 4 (512 threads, one workgroup per CU) up to one tile per CU, else
+     * over 2 (256 threads, two per CU) up to two.  1024^3 f16 with B or A
+     * transposed: 16.9 us on one group and 4 K ranges, 6.4 on four groups;
+     * 1000^3 18.4 and 9.4; 2048^3 with B transposed 29.1 and 22.5.  Ragged and
+     * unaligned matmuls of few tiles, or of one tile row (bound by reading B:
+     * 16 x 8192 x 8192 35.0 us, 35.7 on four groups), and more than twelve
+     * k-steps keep one group and split K across workgroups (plan_gemm_split),
+     * which the SAE encoder does not; over 2 groups they need four k-steps (1400 x 1400 x 136: 6.4 on
+     * one, 6.8 on two). */
+    const bool ksplit = TM_GEMM_KSPLIT && !big &&
+                        (small ? tiles <= 2 * cus : tiles < 2 * cus) &&
+                        p.k >= (whole || tiles <= cus ? 128 : 256) &&
+                        (whole || (small && (!gemm || (4 * tiles > cus && p.m > 64) || p.k <= 768)));
     const int kg = !ksplit ? 1 : small && tiles > cus ? 2 : small ? 4 : 2;
+    /* the kernels that take their K groups from the launch, and their further
+     * groups' LDS (the aligned ones hold one group's tiles themselves); of many
+     * tiles, one group each, the kernel of its own */
+    const bool groups = whole ? !big && !gemm : small;
     plan.variant = format("tm_%s_%s%s%s%s_%s", family,
-                          whole ? "fast" : aligned ? "ragged" : "unaligned", nt ? "_nt" : tn ? "_tn" : "", big ? "" : small ? "_t64" : "_t128",
-                          kg == 4 ? "_k4" : kg == 2 ? "_k2" : "", el);
+                          whole ? "fast" : aligned ? "ragged" : "unaligned", nt ? "_nt" : tn ? "_tn" : "",
+                          big ? "" : small ? "_t64" : "_t128",
+                          groups && kg == 1 && tiles > cus ? "_g1"
+                          : groups                         ? ""
+                          : kg == 4                        ? "_k4"
+                          : kg == 2                        ? "_k2"
+                                                           : "",
+                          el);
     plan.grid[0] = (unsigned)tiles;
     plan.block = (unsigned)(2 * tile * kg);
+    if (groups)
+      plan.lds = (unsigned)((kg - (aligned ? 1 : 0)) * (tile / 64) * TM_GEMM_GROUP_LDS);
     /* whole 256 x 256 tiles: the 4-wave kernel (gemm_w4.hip), whose copies
      * address a step's tile of each operand through one 32-bit buffer range:
      * 256 stored rows of a K-contiguous operand (A row-major, B transposed),
@@ -791,6 +813,7 @@ void choose_gemm(Plan &plan, TmGemmArgs &p, const BuiltinSpec &spec, const char 
     plan.grid[0] = (unsigned)cdiv(p.m, 64);
     plan.grid[1] = (unsigned)cdiv(p.n, 64);
     plan.block = 256;
+    if (spec.element != Element::F32) plan.lds = TM_GEMM_GROUP_LDS;
   }
 }
 
@@ -896,7 +919,12 @@ bool plan_gemm_split(Plan &plan, TmGemmArgs &p, const BuiltinSpec &spec, const L
   const int64_t ksteps = cdiv(p.k, 64);
   const int64_t target = (kg == 1 ? 4 : 1) * cus;
   const int64_t splits = std::min<int64_t>({target / std::max<int64_t>(tiles, 1), ksteps / (2 * kg), 16});
-  if (splits < 2) return false;
+  /* the partials and the reduce dispatch take about as long as eight k-steps of
+   * a wave group (bf16, split and not: 512 x 512 x 2048 saves 6 and runs 9.6 and
+   * 8.7 us, 520 x 776 x 1000 10.8 and 9.5, 512 x 768 x 1536 9.5 and 7.7; at
+   * 512 x 512 x 3072, which saves 9, 10.5 split); of two ranges, half the
+   * partials, as six (200 x 2000 x 3000: 15.0 split, 17.8 not) */
+  if (splits < 2 || (ksteps - ksteps / splits) / kg < (splits == 2 ? 6 : 8)) return false;
   const int64_t np = (p.n + 3) & ~int64_t(3);
   void *work = plan_workspace(lib, (size_t)splits * (size_t)p.m * (size_t)np * 4, scratch);
   if (!work) return false;
@@ -904,10 +932,13 @@ bool plan_gemm_split(Plan &plan, TmGemmArgs &p, const BuiltinSpec &spec, const L
   p.splits = (int32_t)splits;
   Plan main = plan, reduce;
   /* the "_ks" instantiation of the planned kernel */
+  const bool ragged = plan.variant.find("ragged") != std::string::npos;
   const std::string suffix = std::string("_") + el;
-  main.variant = unaligned ? format("tm_gemm_unaligned%s_t64_ks_%s",
-                                    p.layout == TM_GEMM_NT ? "_nt" : p.layout == TM_GEMM_TN ? "_tn" : "", el)
-                           : plan.variant.substr(0, plan.variant.size() - suffix.size()) + "_ks" + suffix;
+  main.variant = unaligned ? format("tm_gemm_unaligned%s_t64",
+                                    p.layout == TM_GEMM_NT ? "_nt" : p.layout == TM_GEMM_TN ? "_tn" : "")
+                           : plan.variant.substr(0, plan.variant.size() - suffix.size());
+  main.variant += (unaligned || ragged) && kg == 4 ? "_k4_ks" + suffix : "_ks" + suffix;
+  main.lds = 0;
   main.grid[1] = (unsigned)splits;
   set_kernarg(main, p);
   reduce.variant = format("tm_gemm_split_reduce_%s", el);
@@ -1460,7 +1491,7 @@ void enqueue(const Plan &plan, hipStream_t stream) {
   if (plan.by_value_struct) {
     void *params[] = {(void *)plan.kernarg.data()};
     hip_check(hipModuleLaunchKernel(plan.function, plan.grid[0], plan.grid[1], plan.grid[2],
-                                    plan.block, 1, 1, 0, stream, params, nullptr),
+                                    plan.block, 1, 1, plan.lds, stream, params, nullptr),
               "hipModuleLaunchKernel");
   } else {
     size_t size = plan.kernarg.size();

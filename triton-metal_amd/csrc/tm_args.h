@@ -20,6 +20,9 @@
 
 /* which strides of A and B are 1: any, both inner ones (row-major), B's along K
  * (B stored transposed), A's along M (A stored transposed) */
+/* LDS of one K group of the 16-bit 64 x 64-tile kernels that take their groups
+ * from the launch (twice it at 128 x 128; the generic any-stride body uses less) */
+#define TM_GEMM_GROUP_LDS 32768
 enum TmGemmLayout { TM_GEMM_ANY = 0, TM_GEMM_NN = 1, TM_GEMM_NT = 2, TM_GEMM_TN = 3 };
 
 struct TmGemmArgs {
