@@ -94,3 +94,24 @@ def test_unaligned_sae(device, element, rows, model, features, kernel):
     got = enc.numpy(x, w, b)
     assert _core.kernel_variant(enc.kernel) == f"tm_sae_{kernel}_{element}"
     assert T.hybrid_error(got, R.sae_encode(x, w, b)) <= 2e-2
+
+
+@pytest.mark.parametrize("m,k", [(2048, 1025), (1 << 20, 1)])
+def test_operand_that_ends_its_allocation(device, m, k):
+    """A fills its buffer.  At 2^20 x 1 that is whole 2 MiB, allocated as asked
+    with nothing behind it, so the loads that reach past the end are not taken;
+    elsewhere the allocation has room for them."""
+    from triton_metal.buffer import DeviceBuffer
+    n = 3
+    rng = np.random.default_rng(3)
+    a = round_to(rng.standard_normal((m, k), dtype=np.float32), "bf16")
+    b = round_to(rng.standard_normal((k, n), dtype=np.float32), "bf16")
+    A, B, C = DeviceBuffer.from_numpy(a, "bfloat16"), DeviceBuffer.from_numpy(b, "bfloat16"), \
+        DeviceBuffer((m, n), "bfloat16")
+    try:
+        ops.matmul(A, B, C, m, n, k)
+        c = C.float32()
+    finally:
+        for x in (A, B, C):
+            x.free()
+    assert T.hybrid_error(c, a.astype(np.float64) @ b.astype(np.float64)) <= 2e-2

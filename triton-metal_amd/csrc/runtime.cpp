@@ -296,6 +296,7 @@ struct Buffer : Object {
   Kind kind() const override { return Kind::Buffer; }
   void *ptr = nullptr;
   int64_t length = 0;
+  int64_t capacity = 0; /* bytes allocated: at least `length` */
   void *host = nullptr; /* the mirror, once tm_buffer_contents was called */
   std::mutex host_lock;
   ~Buffer() override {
@@ -538,6 +539,12 @@ int64_t extent(int64_t rows, int64_t row_stride, int64_t cols, int64_t col_strid
   return e > (__int128)INT64_MAX ? INT64_MAX : (int64_t)e;
 }
 
+/* Whether 14 bytes can be read past the last of `elements` of a 16-bit operand:
+ * the unaligned GEMM kernels' 16-byte loads start at any element. */
+bool has_overhang(const Arg &a, int64_t elements) {
+  return elements <= (a.buffer->capacity - 14) / 2;
+}
+
 /* a + b for non-negative sizes, saturating like extent() */
 int64_t sat_add(int64_t a, int64_t b) { return a > INT64_MAX - b ? INT64_MAX : a + b; }
 
@@ -686,7 +693,8 @@ bool gemm_w4_enabled() {
  * layouts, 16-byte aligned rows and whole 128 x 128 (or, for problems with
  * few of those, 64 x 64) x 32 tiles runs the fp32 MFMA kernel.  Anything else
  * runs the generic 64 x 64 kernel. */
-void choose_gemm(Plan &plan, TmGemmArgs &p, const BuiltinSpec &spec, const char *family) {
+void choose_gemm(Plan &plan, TmGemmArgs &p, const BuiltinSpec &spec, const char *family,
+                 bool overhang) {
   const char *el = element_name(spec.element);
   /* fp32: whole 128 x 128 x 32 tiles on the fp32 MFMA kernel when there are
    * at least half as many of them as compute units, else whole 64 x 64 tiles
@@ -735,9 +743,10 @@ void choose_gemm(Plan &plan, TmGemmArgs &p, const BuiltinSpec &spec, const char 
   const bool a_t8 = a_t && p.sak % 8 == 0, b_t8 = b_t && p.sbn % 8 == 0;
   const bool a_n8 = a_n && p.sam % 8 == 0, b_n8 = b_n && p.sbk % 8 == 0;
   const bool aligned = (a_n8 && (b_n8 || b_t8)) || (a_t8 && b_n8);
-  /* unaligned tiles are addressed by 32-bit byte offsets over up to 256 rows */
+  /* unaligned tiles are addressed by 32-bit byte offsets over up to 256 rows, and
+   * read up to 14 bytes past the operands */
   const int32_t ld_limit = 1 << 22;
-  const bool fits = (p.sak == 1 ? p.sam : p.sak) < ld_limit && (p.sbn == 1 ? p.sbk : p.sbn) < ld_limit;
+  const bool fits = overhang && (p.sak == 1 ? p.sam : p.sak) < ld_limit && (p.sbn == 1 ? p.sbk : p.sbn) < ld_limit;
   const bool nn = aligned ? a_n8 && b_n8 : fits && a_n && b_n;
   const bool nt = !nn && (aligned ? a_n8 && b_t8 : fits && a_n && b_t);
   const bool tn = !nn && !nt && (aligned ? a_t8 && b_n8 : fits && a_t && b_n);
@@ -1041,7 +1050,9 @@ Plan plan_builtin(Kernel &k, const Library &lib, const std::vector<Arg> &args, i
         plan.empty = true;
         return plan;
       }
-      choose_gemm(plan, p, spec, "gemm");
+      choose_gemm(plan, p, spec, "gemm",
+                  has_overhang(args[0], extent(p.m, p.sam, p.k, p.sak)) &&
+                      has_overhang(args[1], extent(p.k, p.sbk, p.n, p.sbn)));
       if (plan_gemm_split(plan, p, spec, lib, scratch)) return plan;
       set_kernarg(plan, p);
       break;
@@ -1076,7 +1087,8 @@ Plan plan_builtin(Kernel &k, const Library &lib, const std::vector<Arg> &args, i
         plan.empty = true;
         return plan;
       }
-      choose_gemm(plan, p, spec, "sae");
+      choose_gemm(plan, p, spec, "sae",
+                  has_overhang(args[0], (int64_t)M * D) && has_overhang(args[1], (int64_t)D * F));
       set_kernarg(plan, p);
       break;
     }
@@ -1877,10 +1889,15 @@ int64_t tm_alloc_buffer(int64_t length) {
   auto buf = std::make_shared<Buffer>();
   /* 16 bytes more than asked for, to whole 256 bytes: the GEMM's 16-byte tile
    * loads may read up to 14 bytes past the end of a matrix whose rows are not a
-   * multiple of 8 elements (those bytes feed only outputs that are not stored). */
+   * multiple of 8 elements (those bytes feed only outputs that are not stored).
+   * Whole multiples of 2 MiB stay what they are (64 MiB + 256 bytes takes the
+   * allocator 29 us and its release 242, 64 MiB 12 and 12); a launch checks for
+   * the room (has_overhang). */
   if (length > INT64_MAX - 271)
     throw TmError(format("could not allocate a %lld-byte device buffer (too large)", (long long)length));
-  hipError_t status = hipMalloc(&buf->ptr, (size_t)((length + 16 + 255) & ~(int64_t)255));
+  const int64_t slack = length % (2 << 20) ? 16 : 0;
+  buf->capacity = (length + slack + 255) & ~(int64_t)255;
+  hipError_t status = hipMalloc(&buf->ptr, (size_t)buf->capacity);
   if (status != hipSuccess) {
     buf->ptr = nullptr;
     (void)hipGetLastError();
