@@ -539,10 +539,10 @@ int64_t extent(int64_t rows, int64_t row_stride, int64_t cols, int64_t col_strid
   return e > (__int128)INT64_MAX ? INT64_MAX : (int64_t)e;
 }
 
-/* Whether 14 bytes can be read past the last of `elements` of a 16-bit operand:
- * the unaligned GEMM kernels' 16-byte loads start at any element. */
-bool has_overhang(const Arg &a, int64_t elements) {
-  return elements <= (a.buffer->capacity - 14) / 2;
+/* Whether 14 bytes can be read past the last of `elements` of an operand: the
+ * GEMM kernels that take rows at any address load 16 bytes from any element. */
+bool has_overhang(const Arg &a, int64_t elements, int element_bytes) {
+  return elements <= (a.buffer->capacity - 14) / element_bytes;
 }
 
 /* a + b for non-negative sizes, saturating like extent() */
@@ -693,6 +693,32 @@ bool gemm_w4_enabled() {
  * layouts, 16-byte aligned rows and whole 128 x 128 (or, for problems with
  * few of those, 64 x 64) x 32 tiles runs the fp32 MFMA kernel.  Anything else
  * runs the generic 64 x 64 kernel. */
+/* fp32 on the bf16 matrix cores (gemm_x3.hip): any M, N, 4-byte aligned rows,
+ * either operand (not both) stored transposed, K past one 32-wide step (below,
+ * the generic kernel: a single step has nothing to overlap).  Whole 16-byte
+ * aligned problems of up to one 128 x 128 tile per compute unit keep the fp32
+ * MFMA kernel, whose K groups suit them (1024^3 22 us, 27 here); more tiles run
+ * here (4096^3: 1050 us there, 725 here).  128 x 128 tiles from half as many as
+ * compute units, else 64 x 64 (1500^3 in 144 tiles and 3 ranges 61 us, in 576 of
+ * 64 x 64 80). */
+bool choose_gemm_x3(Plan &plan, TmGemmArgs &p, const char *family) {
+  const bool gemm = strcmp(family, "gemm") == 0;
+  if (!fast_paths_enabled() || p.scn != 1 || p.k <= 32) return false;
+  const int32_t limit = 1 << 22; /* 32-bit byte offsets over 128 rows */
+  const bool a_n = p.sak == 1 && p.sam >= p.k && p.sam < limit;
+  const bool a_t = !a_n && gemm && p.sam == 1 && p.sak >= p.m && p.sak < limit;
+  const bool b_n = p.sbn == 1 && p.sbk >= p.n && p.sbk < limit;
+  const bool b_t = !b_n && gemm && p.sbk == 1 && p.sbn >= p.k && p.sbn < limit;
+  if (!(a_n && (b_n || b_t)) && !(a_t && b_n)) return false;
+  const int64_t cus = std::max(device().compute_units, 1);
+  const bool big = 2 * cdiv(p.m, 128) * cdiv(p.n, 128) >= cus;
+  const int tile = big ? 128 : 64;
+  plan.variant = format("tm_%s_x3%s%s_f32", family, b_t ? "_nt" : a_t ? "_tn" : "", big ? "" : "_t64");
+  plan.grid[0] = (unsigned)(cdiv(p.m, tile) * cdiv(p.n, tile));
+  plan.block = 256;
+  return true;
+}
+
 void choose_gemm(Plan &plan, TmGemmArgs &p, const BuiltinSpec &spec, const char *family,
                  bool overhang) {
   const char *el = element_name(spec.element);
@@ -709,9 +735,10 @@ void choose_gemm(Plan &plan, TmGemmArgs &p, const BuiltinSpec &spec, const char 
     const bool a_t = gemm && !a_n && p.sam == 1 && p.sak % 4 == 0 && p.sak >= p.m;
     const bool b_n = p.sbn == 1 && p.sbk % 4 == 0 && p.sbk >= p.n;
     const bool b_t = gemm && !b_n && p.sbk == 1 && p.sbn % 4 == 0 && p.sbn >= p.k;
-    if ((a_n || a_t) && (b_n || b_t) && !(a_t && b_t)) {
-      const int tile = f32_big ? 128 : 64;
-      const int64_t tiles = (int64_t)(p.m / tile) * (p.n / tile);
+    const int tile = f32_big ? 128 : 64;
+    const int64_t tiles = (int64_t)(p.m / tile) * (p.n / tile);
+    if ((a_n || a_t) && (b_n || b_t) && !(a_t && b_t) &&
+        !(f32_big && tiles > device().compute_units && choose_gemm_x3(plan, p, family))) {
       /* About one workgroup per CU or fewer (one wave per SIMD): split the K
        * loop over 2 (128 x 128 tiles) or up to 4 (64 x 64) groups of waves
        * inside the workgroup (plain row-major matmul only) */
@@ -727,7 +754,9 @@ void choose_gemm(Plan &plan, TmGemmArgs &p, const BuiltinSpec &spec, const char 
       plan.block = (unsigned)(256 * kg);
       return;
     }
+    if (plan.block) return; /* the x3 kernel */
   }
+  if (spec.element == Element::F32 && overhang && choose_gemm_x3(plan, p, family)) return;
   const bool half = fast_paths_enabled() && spec.element != Element::F32 && p.scn == 1 && p.k > 0;
   /* A row-major [M, K], or (matmul only) stored transposed: element (m, k) at
    * k * stride_ak + m, the dY^T X layout */
@@ -963,6 +992,39 @@ bool plan_gemm_split(Plan &plan, TmGemmArgs &p, const BuiltinSpec &spec, const L
 }
 
 
+/* The split of an x3 GEMM's k-steps into ranges (grid y), likewise, for the SAE
+ * encoder too: its epilogue moves to the reduce dispatch. */
+bool plan_x3_split(Plan &plan, TmGemmArgs &p, const Library &lib, const Scratch *scratch) {
+  if (plan.variant.find("_x3") == std::string::npos) return false;
+  const int64_t cus = std::max(device().compute_units, 1);
+  const int64_t tiles = plan.grid[0], ksteps = cdiv(p.k, 32);
+  const bool small = plan.variant.find("_t64") != std::string::npos;
+  /* two workgroups of 128 x 128 tiles or four of 64 x 64 per compute unit, at
+   * least four steps to a range (fp32, us without ranges and with: 500^3 18.4
+   * and 11.7, 1000^3 36 and 28, 64 x 1088 x 5504 111 on the generic kernel and
+   * 21, SAE 24 x 3856 x 12352 110 and 55) */
+  const int64_t target = (small ? 4 : 2) * cus;
+  const int64_t splits = std::min<int64_t>({target / tiles, ksteps / 4, 16});
+  if (splits < 2) return false;
+  const int64_t np = (p.n + 3) & ~int64_t(3);
+  void *work = plan_workspace(lib, (size_t)splits * (size_t)p.m * (size_t)np * 4, scratch);
+  if (!work) return false;
+  p.part = (float *)work;
+  p.splits = (int32_t)splits;
+  Plan main = plan, reduce;
+  main.grid[1] = (unsigned)splits;
+  set_kernarg(main, p);
+  reduce.variant = plan.variant.compare(0, 6, "tm_sae") == 0 ? "tm_sae_split_reduce_f32" : "tm_gemm_split_reduce_f32";
+  reduce.grid[0] = (unsigned)cdiv((int64_t)p.m * (np / 4), 256);
+  reduce.block = 256;
+  set_kernarg(reduce, p);
+  for (Plan *part : {&main, &reduce}) part->function = builtin_function(part->variant);
+  plan.function = main.function;
+  plan.variant = format("%s + %s (%d K ranges)", main.variant.c_str(), reduce.variant.c_str(), (int)splits);
+  plan.sequence = {main, reduce};
+  return true;
+}
+
 /* Ranges to split a generic attention kernel's walk into when its grid of
  * `wgs` 64-row workgroups cannot fill the chip twice: enough to (at most 16,
  * each at least two 32-row blocks of the `n_ctx` walked); 1 for no split. */
@@ -1051,9 +1113,9 @@ Plan plan_builtin(Kernel &k, const Library &lib, const std::vector<Arg> &args, i
         return plan;
       }
       choose_gemm(plan, p, spec, "gemm",
-                  has_overhang(args[0], extent(p.m, p.sam, p.k, p.sak)) &&
-                      has_overhang(args[1], extent(p.k, p.sbk, p.n, p.sbn)));
-      if (plan_gemm_split(plan, p, spec, lib, scratch)) return plan;
+                  has_overhang(args[0], extent(p.m, p.sam, p.k, p.sak), es) &&
+                      has_overhang(args[1], extent(p.k, p.sbk, p.n, p.sbn), es));
+      if (plan_gemm_split(plan, p, spec, lib, scratch) || plan_x3_split(plan, p, lib, scratch)) return plan;
       set_kernarg(plan, p);
       break;
     }
@@ -1088,7 +1150,8 @@ Plan plan_builtin(Kernel &k, const Library &lib, const std::vector<Arg> &args, i
         return plan;
       }
       choose_gemm(plan, p, spec, "sae",
-                  has_overhang(args[0], (int64_t)M * D) && has_overhang(args[1], (int64_t)D * F));
+                  has_overhang(args[0], (int64_t)M * D, es) && has_overhang(args[1], (int64_t)D * F, es));
+      if (plan_x3_split(plan, p, lib, scratch)) return plan;
       set_kernarg(plan, p);
       break;
     }
