@@ -52,6 +52,9 @@ def _check(c, a, b, k):
     (1409, 1281, 161, 1, ""),          # 12 x 11 tiles of 128, K ranges
     (2177, 2050, 95, 1, ""),           # 18 x 17 tiles
     (2304, 2176, 64, 0, ""),           # whole tiles, more than one per compute unit
+    (2048, 1024, 1056, 0, ""),         # whole 128 x 128 tiles for half of them, long K
+    (128, 320, 512, 0, "_t64"),        # whole 64 x 64 tiles, few
+    (1088, 1024, 768, 0, "_t64"),      # and more than one per compute unit
 ])
 def test_x3_gemm(device, layout, m, n, k, pad, kernel):
     rng = np.random.default_rng(m + n + k)

@@ -695,10 +695,7 @@ bool gemm_w4_enabled() {
  * runs the generic 64 x 64 kernel. */
 /* fp32 on the bf16 matrix cores (gemm_x3.hip): any M, N, 4-byte aligned rows,
  * either operand (not both) stored transposed, K past one 32-wide step (below,
- * the generic kernel: a single step has nothing to overlap).  Whole 16-byte
- * aligned problems of up to one 128 x 128 tile per compute unit keep the fp32
- * MFMA kernel, whose K groups suit them (1024^3 22 us, 27 here); more tiles run
- * here (4096^3: 1050 us there, 725 here).  128 x 128 tiles from half as many as
+ * the generic kernel: a single step has nothing to overlap).  128 x 128 tiles from half as many as
  * compute units, else 64 x 64 (1500^3 in 144 tiles and 3 ranges 61 us, in 576 of
  * 64 x 64 80). */
 bool choose_gemm_x3(Plan &plan, TmGemmArgs &p, const char *family) {
@@ -737,14 +734,23 @@ void choose_gemm(Plan &plan, TmGemmArgs &p, const BuiltinSpec &spec, const char 
     const bool b_t = gemm && !b_n && p.sbk == 1 && p.sbn % 4 == 0 && p.sbn >= p.k;
     const int tile = f32_big ? 128 : 64;
     const int64_t tiles = (int64_t)(p.m / tile) * (p.n / tile);
-    if ((a_n || a_t) && (b_n || b_t) && !(a_t && b_t) &&
-        !(f32_big && tiles > device().compute_units && choose_gemm_x3(plan, p, family))) {
+    /* the bf16-split kernel (whole tiles of 16-byte aligned rows leave it nothing
+     * to read past an operand), us against this one's: more 128 x 128 tiles than
+     * compute units 725 / 1050 (4096^3); up to as many, past K = 1024, 109 / 134
+     * (2048 x 2048 x 1984), 64 / 135 (2048 x 1024 x 2016, B transposed); 64 x 64
+     * tiles for half the compute units, from K = 512 in ranges, 16 / 23 (512 x
+     * 512 x 992), 23 / 111 (64 x 1088 x 5504), or for more than all of them 31 / 38
+     * (1088 x 1024 x 992; at K = 512 23 / 21); between, 28 / 23 (1024 x 1024 x
+     * 992) */
+    const int64_t cus = std::max(device().compute_units, 1);
+    const bool x3 = f32_big ? tiles > cus || p.k > 1024
+                            : 2 * tiles <= cus ? p.k >= 512 : tiles > cus && p.k >= 768;
+    if ((a_n || a_t) && (b_n || b_t) && !(a_t && b_t) && !(x3 && choose_gemm_x3(plan, p, family))) {
       /* About one workgroup per CU or fewer (one wave per SIMD): split the K
        * loop over 2 (128 x 128 tiles) or up to 4 (64 x 64) groups of waves
        * inside the workgroup (plain row-major matmul only) */
       int64_t kg = 1;
       if (gemm && a_n && b_n) {
-        const int64_t cus = std::max(device().compute_units, 1);
         kg = std::min<int64_t>({2 * cus / std::max<int64_t>(tiles, 1), f32_big ? 2 : 4, p.k / 32});
         kg = kg >= 4 ? 4 : kg >= 2 ? 2 : 1;
       }
