@@ -1,0 +1,81 @@
+"""fp32 attention on the bf16 matrix cores (three-way split operands): block and
+head-dimension edges, odd strides, and values that the split cannot hold, which
+the generic body computes, all at the fp32 tests' bounds."""
+
+import math
+
+import numpy as np
+import pytest
+
+from oracle import reference as R
+from oracle import tolerance as T
+from test_fast_paths_gpu import _attention
+from triton_metal import ops
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("causal", [False, True])
+@pytest.mark.parametrize("heads,seq,dim,pad", [
+    (2, 1, 64, 0), (2, 63, 64, 1), (3, 65, 64, 3), (1, 130, 33, 0), (2, 97, 5, 2), (2, 31, 96, 1),
+    (1, 33, 127, 0), (9, 200, 128, 4), (40, 520, 64, 0), (70, 130, 32, 0),
+])
+def test_edges(device, heads, seq, dim, pad, causal):
+    """Head dimensions that are no multiple of 8, rows at any 4-byte address,
+    split (few heads) and whole walks."""
+    out, variants, dense, _ = _attention(heads, seq, dim, "f32", causal, stride_seq=dim + pad)
+    assert "_generic_f32_d" in variants[0]
+    want = R.attention_backward(*dense, 1 / math.sqrt(dim), causal)
+    assert T.hybrid_error(out["o"], want["o"]) <= 2e-5
+    assert T.hybrid_error(out["lse"], want["lse"]) <= 2e-5
+    for name in ("dq", "dk", "dv"):
+        assert T.hybrid_error(out[name], want[name]) <= 1e-4, name
+
+
+def _layer(x, scale, causal=False):
+    heads, seq, dim = x["q"].shape
+    layer = ops.AttentionLayer(heads, seq, dim, "f32", causal, scale=scale)
+    try:
+        o, lse = layer.forward(x["q"], x["k"], x["v"])
+        dq, dk, dv = layer.backward(x["do"])
+    finally:
+        layer.free()
+    return {"o": o, "lse": lse, "dq": dq, "dk": dk, "dv": dv}
+
+
+def _inputs(heads=2, seq=150, dim=64, seed=3):
+    rng = np.random.default_rng(seed)
+    return {n: rng.standard_normal((heads, seq, dim), dtype=np.float32) for n in ("q", "k", "v", "do")}
+
+
+@pytest.mark.parametrize("name,power", [("k", -110), ("q", -115), ("v", -105), ("do", -108)])
+def test_values_below_the_split(device, name, power):
+    """One tensor near the bottom of the range: gradients and outputs scale with
+    it exactly as at 1 (a power of two), within the same bounds."""
+    x = _inputs()
+    scale = 1 / 8.0
+    want = R.attention_backward(x["q"], x["k"], x["v"], x["do"], scale, False)
+    x[name] = np.ldexp(x[name], power)
+    if name in ("q", "k"):
+        other = "k" if name == "q" else "q"
+        x[other] = np.ldexp(x[other], -power)
+    got = _layer(x, scale)
+    powers = {"k": {"dq": power, "dk": -power}, "q": {"dk": power, "dq": -power},
+              "v": {"o": power, "dq": power, "dk": power},
+              "do": {"dq": power, "dk": power, "dv": power}}[name]
+    for out in ("o", "lse", "dq", "dk", "dv"):
+        back = np.ldexp(got[out].astype(np.float64), -powers.get(out, 0))
+        assert T.hybrid_error(back, want[out]) <= 1e-4, out
+
+
+def test_infinities_stay_in_their_columns(device):
+    x = _inputs(seq=100)
+    x["v"][0, 7, 3] = np.inf
+    got = _layer(x, 1 / 8.0)
+    x["v"][0, 7, 3] = 0.0
+    want, _, _ = R.attention_forward(x["q"], x["k"], x["v"], 1 / 8.0, False)
+    assert np.all(got["o"][0, :, 3] == np.inf)
+    keep = np.ones(64, bool)
+    keep[3] = False
+    assert T.hybrid_error(got["o"][0][:, keep], want[0][:, keep]) <= 2e-5
+    assert T.hybrid_error(got["o"][1], want[1]) <= 2e-5

@@ -23,20 +23,13 @@
  * v_mfma_f32_16x16x4_f32, straight from memory.
  */
 #include "gemm_fast.h"
+#include "split3.h"
 
 namespace {
 
 constexpr int XK = 32; /* k per step */
 
 typedef f32x4 f32x4_any __attribute__((aligned(4)));
-
-/* two floats -> their bf16 roundings in one word, and what the roundings leave */
-TM_DEV uint32_t x3_part(float &a, float &b) {
-  const uint32_t w = g_pack2<bf16_t>(a, b);
-  a -= __uint_as_float(w << 16);
-  b -= __uint_as_float(w & 0xffff0000u);
-  return w;
-}
 
 /* A [TILE rows][32 k] plane (k contiguous): 64-byte rows of four 16-byte chunks,
  * chunk c of row r at c ^ ((r >> 2) & 3): 16 rows at one chunk (ds_read_b128 of
@@ -107,8 +100,7 @@ struct X3Tile {
             if (chunk * 8 + h * 4 + e >= width) v[t][h][e] = 0.f;
     }
   }
-  /* split into the planes at `lds`; `least` keeps the smallest nonzero magnitude
-   * seen (twice its bits, less one) */
+  /* split into the planes at `lds` */
   TM_DEV void store(char *lds, uint32_t &least) {
 #pragma unroll
     for (int t = 0; t < TASKS; ++t) {
@@ -118,15 +110,12 @@ struct X3Tile {
 #pragma unroll
       for (int e = 0; e < 8; ++e) {
         x[e] = v[t][e >> 2][e & 3];
-        least = min(least, (__float_as_uint(x[e]) << 1) - 1u);
+        least = x3_least(least, x[e]);
       }
+      u32x4 part[3];
+      x3_split8(x, part);
 #pragma unroll
-      for (int q = 0; q < 3; ++q) {
-        u32x4 w;
-#pragma unroll
-        for (int e = 0; e < 4; ++e) w[e] = x3_part(x[2 * e], x[2 * e + 1]);
-        *(u32x4 *)(lds + q * PLANE + at) = w;
-      }
+      for (int q = 0; q < 3; ++q) *(u32x4 *)(lds + q * PLANE + at) = part[q];
     }
   }
 };
@@ -182,7 +171,7 @@ TM_DEV void gemm_x3(const TmGemmArgs &p) {
   for (int i = 0; i < NI; ++i)
 #pragma unroll
     for (int j = 0; j < NI; ++j) acc[i][j] = (f32x4){0.f, 0.f, 0.f, 0.f};
-  uint32_t least = 0xffffffffu;
+  uint32_t least = X3_NONE;
 
   if (kbeg < kend) load(kbeg);
   for (int kb = kbeg; kb < kend; ++kb) {
@@ -222,15 +211,13 @@ TM_DEV void gemm_x3(const TmGemmArgs &p) {
     __syncthreads();
   }
 
-  /* beyond the split: twice the bits of 2^-100, less one; or anything that is
-   * not finite (its difference from itself is not zero) */
-  bool beyond = least < ((27u << 24) - 1u);
+  bool beyond = x3_below(least);
 #pragma unroll
   for (int i = 0; i < NI; ++i)
 #pragma unroll
     for (int j = 0; j < NI; ++j)
 #pragma unroll
-      for (int r = 0; r < 4; ++r) beyond |= !(acc[i][j][r] - acc[i][j][r] == 0.f);
+      for (int r = 0; r < 4; ++r) beyond |= x3_not_finite(acc[i][j][r]);
   if (__syncthreads_or(beyond)) {
     const int kstop = min(p.k, kend * XK);
 #pragma unroll
