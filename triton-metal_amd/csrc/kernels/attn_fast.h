@@ -758,7 +758,7 @@ TM_DEV void attn_pre_fast(const TmAttnPreArgs &p) {
  * branch between the two buffer phases in the masked loop) the kernel needed
  * 256 registers and spilled; so it needs 234 and runs 3% faster. */
 template <int D> struct DqLds { static constexpr int BYTES = 4 * 64 * D * 2; };
-template <typename T, int D, bool CAUSAL, int DC = D, bool PAD = false>
+template <typename T, int D, bool CAUSAL, int DC = D, bool PAD = false, bool RANGES = false>
 TM_DEV void attn_dq_fast(const TmAttnDqArgs &p, char *lds, int wg, int nwg) {
   constexpr int BM = 128, BN = 64, QW = 32;
   constexpr int KS = (DC + 31) / 32, DT = DC / 16;
@@ -793,14 +793,18 @@ TM_DEV void attn_dq_fast(const TmAttnDqArgs &p, char *lds, int wg, int nwg) {
   const float *Dg = p.delta + (int64_t)bh * p.stride_lse;
 
   const int kend = CAUSAL ? min(n, q0 + BM) : n;
-  const int nblocks = (kend + BN - 1) / BN;
+  const int all_blocks = (kend + BN - 1) / BN;
+  /* the key blocks this workgroup walks: all of them, or (RANGES) the z-th of
+   * p.splits contiguous ranges */
+  const int first = RANGES ? (int)blockIdx.z * all_blocks / p.splits : 0;
+  const int nblocks = RANGES ? ((int)blockIdx.z + 1) * all_blocks / p.splits : all_blocks;
   TileCopy<T, D, BN, KEY_BOTH> kvcp; /* K and V rows share the lane offsets */
   const int chunks = PAD ? p.head_dim / 8 : D / 8;
   if constexpr (PAD) kvcp.init_padded(ss, wave, lane, p.head_dim);
   else kvcp.init(ss, wave, lane);
-  if (nblocks > 0) {
-    kvcp.copy(Kg, ss, 0, n, buf_a, wave);
-    kvcp.copy(Vg, ss, 0, n, buf_a + TILE, wave);
+  if (nblocks > first) {
+    kvcp.copy(Kg, ss, first * BN, n, buf_a, wave);
+    kvcp.copy(Vg, ss, first * BN, n, buf_a + TILE, wave);
   }
   /* lane parts of the operand offsets (row offsets of kt are immediates) */
   uint32_t koff[KS], kmoff[DT];
@@ -896,13 +900,15 @@ TM_DEV void attn_dq_fast(const TmAttnDqArgs &p, char *lds, int wg, int nwg) {
   using Interior = std::integral_constant<bool, false>;
   using Edge = std::integral_constant<bool, true>;
 
-  const int n_interior = CAUSAL ? min(q0 / BN, n / BN) : n / BN;
-  int j = 0;
+  const int n_unmasked = CAUSAL ? min(q0 / BN, n / BN) : n / BN;
+  const int n_interior = RANGES ? min(n_unmasked, nblocks) : n_unmasked;
+  int j = first;
   for (; j + 1 < n_interior; j += 2) {
     step(Interior{}, buf_a, buf_b, j);
     step(Interior{}, buf_b, buf_a, j + 1);
   }
-  for (; j < nblocks; ++j) step(Edge{}, (j & 1) ? buf_b : buf_a, (j & 1) ? buf_a : buf_b, j);
+  for (; j < nblocks; ++j)
+    step(Edge{}, ((j - first) & 1) ? buf_b : buf_a, ((j - first) & 1) ? buf_a : buf_b, j);
 
 #pragma unroll
   for (int qt = 0; qt < 2; ++qt) {
@@ -911,6 +917,11 @@ TM_DEV void attn_dq_fast(const TmAttnDqArgs &p, char *lds, int wg, int nwg) {
 #pragma unroll
       for (int dt = 0; dt < DT; ++dt) {
         if (PAD && dt * 16 + 4 * g >= p.head_dim) continue;
+        if constexpr (RANGES) {
+          float *part = p.part + (((int64_t)blockIdx.z * p.heads + bh) * n + qi) * p.head_dim;
+          *(f32x4 *)(part + dt * 16 + 4 * g) = acc[dt][qt];
+          continue;
+        }
         u32x2 w;
         w[0] = pack2<T>(acc[dt][qt][0] * p.sm_scale, acc[dt][qt][1] * p.sm_scale);
         w[1] = pack2<T>(acc[dt][qt][2] * p.sm_scale, acc[dt][qt][3] * p.sm_scale);
@@ -1302,7 +1313,7 @@ template <int D> struct Dkdv2wLds {
   static constexpr int BM = D == 64 ? 64 : 32; /* query rows per copied block */
   static constexpr int BYTES = 128 * D * 2 + 2 * (2 * BM * D * 2 + BM * 8);
 };
-template <typename T, int D, bool CAUSAL, int DC = D, bool PAD = false>
+template <typename T, int D, bool CAUSAL, int DC = D, bool PAD = false, bool RANGES = false>
 TM_DEV void attn_dkdv_2w(const TmAttnDkdvArgs &p, char *lds, int wg, int nwg) {
   constexpr int BN = 128, KW = 32, BM = Dkdv2wLds<D>::BM;
   constexpr int KS = (DC + 31) / 32, DT = DC / 16;
@@ -1341,7 +1352,11 @@ TM_DEV void attn_dkdv_2w(const TmAttnDkdvArgs &p, char *lds, int wg, int nwg) {
   const float *Dg = p.delta + (int64_t)bh * p.stride_lse;
 
   const int q_start = CAUSAL ? k0 : 0;
-  const int nblocks = (n - q_start + BM - 1) / BM;
+  const int all_blocks = (n - q_start + BM - 1) / BM;
+  /* the query blocks this workgroup walks: all of them, or (RANGES) the z-th of
+   * p.splits contiguous ranges */
+  const int first = RANGES ? (int)blockIdx.z * all_blocks / p.splits : 0;
+  const int nblocks = RANGES ? ((int)blockIdx.z + 1) * all_blocks / p.splits : all_blocks;
 
   TileCopy<T, D, BM, KEY_BOTH> qcp;  /* Q and dO rows share the lane offsets */
   TileCopy<T, D, BN, KEY_B128> vcp;
@@ -1363,7 +1378,7 @@ TM_DEV void attn_dkdv_2w(const TmAttnDkdvArgs &p, char *lds, int wg, int nwg) {
     }
   };
   vcp.copy(Vg, ss, k0, n, vbase, wave);
-  if (nblocks > 0) stage(buf0, 0);
+  if (nblocks > first) stage(buf0, first);
 
   u32x4 kf[2][KS];
 #pragma unroll
@@ -1478,7 +1493,8 @@ TM_DEV void attn_dkdv_2w(const TmAttnDkdvArgs &p, char *lds, int wg, int nwg) {
    * the masked blocks (the diagonal band, a ragged end) and the interior run
    * in loops of their own */
   auto step = [&](auto edge_tag, int i) {
-    const uint32_t cur = (i & 1) ? buf1 : buf0, nxt = (i & 1) ? buf0 : buf1;
+    const bool odd = (i - first) & 1;
+    const uint32_t cur = odd ? buf1 : buf0, nxt = odd ? buf0 : buf1;
     if (i + 1 < nblocks) stage(nxt, i + 1);
     /* causal: a block whose every query precedes the wave's first key adds
      * exact zeros; the wave skips its arithmetic (not its copies and barrier),
@@ -1490,7 +1506,7 @@ TM_DEV void attn_dkdv_2w(const TmAttnDkdvArgs &p, char *lds, int wg, int nwg) {
     __syncthreads();
   };
   const int interior_end = min(full, nblocks);
-  int i = 0;
+  int i = first;
   for (; i < nblocks && i < band; ++i) step(Edge{}, i);
   for (; i < interior_end; ++i) step(Interior{}, i);
   for (; i < nblocks; ++i) step(Edge{}, i);
@@ -1503,6 +1519,13 @@ TM_DEV void attn_dkdv_2w(const TmAttnDkdvArgs &p, char *lds, int wg, int nwg) {
 #pragma unroll
       for (int dt = 0; dt < DT; ++dt) {
         if (PAD && dt * 16 + 4 * g >= p.head_dim) continue;
+        if constexpr (RANGES) {
+          const int64_t plane = (int64_t)p.heads * n * p.head_dim;
+          float *part = p.part + 2 * (int64_t)blockIdx.z * plane + ((int64_t)bh * n + key) * p.head_dim;
+          *(f32x4 *)(part + dt * 16 + 4 * g) = -dk[dt][kt];
+          *(f32x4 *)(part + plane + dt * 16 + 4 * g) = dv[dt][kt];
+          continue;
+        }
         u32x2 wk, wv;
         wk[0] = pack2<T>(dk[dt][kt][0] * dk_scale, dk[dt][kt][1] * dk_scale);
         wk[1] = pack2<T>(dk[dt][kt][2] * dk_scale, dk[dt][kt][3] * dk_scale);

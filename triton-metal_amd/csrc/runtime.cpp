@@ -1040,16 +1040,31 @@ int64_t split_ranges(int64_t wgs, int64_t n_ctx) {
   return std::max<int64_t>(1, std::min<int64_t>({cdiv(2 * cus, wgs), cdiv(n_ctx, 32) / 2, 16}));
 }
 
+/* The same for the 16-bit dq and dkdv kernels, `wgs` workgroups of 128 rows:
+ * ranges of at least 256 rows, up to two workgroups per compute unit, where the
+ * walk saved is longer than the reduce dispatch: from 768 rows for an eighth as
+ * many workgroups as compute units, up to a quarter at more than 64 columns or
+ * from 1536 rows.  bf16, dQ + dK/dV whole and in ranges, us: 1 head x 1000 x 64 43
+ * and 29, 1 x 4000 144 and 51, 4 x 2048 78 and 60, 8 x 1024 43 and 44 (at 128
+ * columns causal 73 and 53); 16 x 1000 44 and 66. */
+int64_t fast_ranges(int64_t wgs, int64_t n_ctx, int head_dim) {
+  const int64_t cus = std::max(device().compute_units, 1);
+  const bool worth = 8 * wgs <= cus || (4 * wgs <= cus && (head_dim > 64 || n_ctx >= 1536));
+  if (n_ctx < 768 || !worth) return 1;
+  return std::max<int64_t>(1, std::min<int64_t>({2 * cus / wgs, n_ctx / 256, 16}));
+}
+
 /* The split form of a generic dq or dkdv plan: the main dispatch over
  * `splits` ranges (grid z) writing fp32 partials to `part`, then the reduce
  * dispatch that sums them into the outputs (dQ * sm_scale, or dK * sm_scale
  * and dV) in the element type. */
 template <typename A>
 void plan_split_backward(Plan &plan, const BuiltinSpec &spec, A p, float *part, int64_t splits,
-                         void *out0, void *out1) {
+                         bool fast, void *out0, void *out1) {
   p.part = part;
   p.splits = (int32_t)splits;
   Plan main = plan, reduce;
+  if (fast) main.variant += "_ranges";
   main.grid[2] = (unsigned)splits;
   set_kernarg(main, p);
   TmAttnSplitReduceArgs r{};
@@ -1336,13 +1351,14 @@ Plan plan_builtin(Kernel &k, const Library &lib, const std::vector<Arg> &args, i
         p.head_dim = spec.head_dim;
         p.heads = (int32_t)heads;
         plan.variant = fast ? fast_name : attn_symbol("dq", spec);
-        const int64_t splits = fast ? 1 : split_ranges((int64_t)plan.grid[0] * heads, n_ctx);
+        const int64_t splits = fast ? fast_ranges(plan.grid[0], n_ctx, spec.head_dim)
+                                    : split_ranges((int64_t)plan.grid[0] * heads, n_ctx);
         void *work = splits > 1 ? plan_workspace(lib, (size_t)splits * (size_t)heads * (size_t)n_ctx *
                                                           (size_t)spec.head_dim * 4,
                                                  scratch)
                                 : nullptr;
         if (work) {
-          plan_split_backward(plan, spec, p, (float *)work, splits, p.dq, nullptr);
+          plan_split_backward(plan, spec, p, (float *)work, splits, fast, p.dq, nullptr);
           return plan;
         }
         set_kernarg(plan, p);
@@ -1364,13 +1380,14 @@ Plan plan_builtin(Kernel &k, const Library &lib, const std::vector<Arg> &args, i
         p.head_dim = spec.head_dim;
         p.heads = (int32_t)heads;
         plan.variant = fast ? fast_name : attn_symbol("dkdv", spec);
-        const int64_t splits = fast ? 1 : split_ranges((int64_t)plan.grid[0] * heads, n_ctx);
+        const int64_t splits = fast ? fast_ranges(plan.grid[0], n_ctx, spec.head_dim)
+                                    : split_ranges((int64_t)plan.grid[0] * heads, n_ctx);
         void *work = splits > 1 ? plan_workspace(lib, (size_t)splits * 2 * (size_t)heads *
                                                           (size_t)n_ctx * (size_t)spec.head_dim * 4,
                                                  scratch)
                                 : nullptr;
         if (work) {
-          plan_split_backward(plan, spec, p, (float *)work, splits, p.dk, p.dv);
+          plan_split_backward(plan, spec, p, (float *)work, splits, fast, p.dk, p.dv);
           return plan;
         }
         set_kernarg(plan, p);
