@@ -931,7 +931,8 @@ TM_DEV void attn_dq_fast(const TmAttnDqArgs &p, char *lds, int wg, int nwg) {
   }
 }
 
-/* ---- backward: dK, dV and dQ in one pass (bwd=atomic) -----------------------
+/* ---- backward: dK, dV with one wave per SIMD, and (FUSED, bwd=atomic) dQ in the
+ * same pass ------------------------------------------------------------------
  * One workgroup = 4 waves = 128 keys; each wave owns 32 keys, held in
  * registers (K^T and V^T as B operands), and walks the query blocks (BM = 32
  * queries at D = 128, 64 at D = 64) of its head.  Per block, with the lane owning one key:
@@ -950,15 +951,15 @@ TM_DEV void attn_dq_fast(const TmAttnDqArgs &p, char *lds, int wg, int nwg) {
  * are independent, so the wave's VALU work overlaps its MFMA work.  Buffer
  * indices are compile-time (PH = i mod 3) so the compiler sees that the
  * in-flight copy never aliases the tiles being read. */
-template <typename T, int D, bool CAUSAL>
-TM_DEV void attn_bwd_fused(const TmAttnDkdvArgs &p, float *dq_acc) {
+template <typename T, int D, bool CAUSAL, bool FUSED>
+TM_DEV void attn_dkdv_1w(const TmAttnDkdvArgs &p, float *dq_acc = nullptr) {
   /* query rows per step: 64 at D = 64 (twice the MFMA work per barrier and
    * per softmax pass; measured 7% faster), 32 at D = 128, where 64 would not
    * fit the registers */
   constexpr int BN = 128, KW = 32, BM = D == 64 ? 64 : 32;
   /* The kernel carries -dS = P (Delta - dP): the dP MFMAs run on -V and start
    * from Delta, so no subtraction per element.  dK accumulates -dK and flips
-   * the sign at the store; dQ is added with -K. */
+   * the sign at the store; FUSED adds dQ with -K. */
   constexpr int QT = BM / 16, KK = BM / 32;
   constexpr int KS = D / 32;
   constexpr int TILE = BM * D * 2;
@@ -967,10 +968,10 @@ TM_DEV void attn_bwd_fused(const TmAttnDkdvArgs &p, float *dq_acc) {
   __shared__ __align__(1024) char lds_0[BUF];
   __shared__ __align__(1024) char lds_1[BUF];
   __shared__ __align__(1024) char lds_2[BUF];
-  /* dS of two query blocks, [BN keys][BM queries] each, so that every
+  /* FUSED: dS of two query blocks, [BN keys][BM queries] each, so that every
    * wave can read all 128 keys of it (ds_off) */
   constexpr int DS_TILE = BN * BM * 2;
-  __shared__ __align__(1024) char lds_ds[2 * DS_TILE];
+  __shared__ __align__(1024) char lds_ds[FUSED ? 2 * DS_TILE : 16];
 
   typedef typename Vec8<T>::type v8;
   const int tid = threadIdx.x, lane = tid & 63;
@@ -1021,14 +1022,14 @@ TM_DEV void attn_bwd_fused(const TmAttnDkdvArgs &p, float *dq_acc) {
       vf[kt][ks] ^= (u32x4){0x80008000u, 0x80008000u, 0x80008000u, 0x80008000u};
     }
   }
-  /* K as the B operand of dQ[:, wave's D/4 columns] = dS K, for the
+  /* FUSED: K as the B operand of dQ[:, wave's D/4 columns] = dS K, for the
    * 128 keys in four 32-key steps; element j of a lane holds key
    * 32 ks + 4g + j (j < 4) or 32 ks + 16 + 4g + j - 4, the order in which the
    * transposing read of dS delivers them.  Keys at or past n are zero, so the
    * (finite) dS of those padding keys adds nothing. */
-  constexpr int NT = D / 64;
-  u32x4 kq[4][NT];
-  {
+  constexpr int NT = FUSED ? D / 64 : 1;
+  u32x4 kq[FUSED ? 4 : 1][NT];
+  if constexpr (FUSED) {
     const uint16_t *Kh = (const uint16_t *)Kg;
 #pragma unroll
     for (int ks = 0; ks < 4; ++ks)
@@ -1130,7 +1131,7 @@ TM_DEV void attn_bwd_fused(const TmAttnDkdvArgs &p, float *dq_acc) {
     }
   };
 
-  /* byte offset of queries q .. q+3 (q a multiple of 4) of key row
+  /* FUSED: byte offset of queries q .. q+3 (q a multiple of 4) of key row
    * `key` in a dS tile; 16-byte chunks XOR-swizzled so that the 16 rows one
    * transposing read spans fall on distinct banks */
   auto ds_off = [&](int key, int q) {
@@ -1201,10 +1202,10 @@ TM_DEV void attn_bwd_fused(const TmAttnDkdvArgs &p, float *dq_acc) {
     u32x4 pf2[2][KK], ds2[2][KK];
     if (!CHECKED || i + 1 < nblocks) {
       scores(edge_tag, nx1, i + 1, pf2, ds2);
-      put_ds(i + 1, ds2);
+      if constexpr (FUSED) put_ds(i + 1, ds2);
     }
     grads(cur, pf, dsf);
-    dq_block(i);
+    if constexpr (FUSED) dq_block(i);
 #pragma unroll
     for (int kt = 0; kt < 2; ++kt)
 #pragma unroll
@@ -1240,8 +1241,10 @@ TM_DEV void attn_bwd_fused(const TmAttnDkdvArgs &p, float *dq_acc) {
   wait_vmem();
   __syncthreads();
   if (nblocks > 0) scores(Edge{}, lds_0, 0, pf, dsf);
-  if (nblocks > 0) put_ds(0, dsf);
-  __syncthreads();
+  if constexpr (FUSED) {
+    if (nblocks > 0) put_ds(0, dsf);
+    __syncthreads();
+  }
 
   /* Block b is masked if it lies in the diagonal band (b < band) or runs past
    * n (b >= full).  Step i masks the softmax of block i+1. */
@@ -1286,7 +1289,7 @@ TM_DEV void attn_bwd_fused(const TmAttnDkdvArgs &p, float *dq_acc) {
 
 
 /* ---- backward: dK, dV ------------------------------------------------------
- * The work split of attn_bwd_fused (a workgroup of 4 waves owns 128 keys, a wave
+ * The work split of attn_dkdv_1w (a workgroup of 4 waves owns 128 keys, a wave
  * 32 of them) without dQ, built for two waves per SIMD (three at D = 64) so that
  * the other workgroup's wave fills the MFMA pipe while this one runs its
  * softmax.  To fit 256 registers the wave keeps only K^T in registers; the
@@ -1305,7 +1308,7 @@ TM_DEV void attn_bwd_fused(const TmAttnDkdvArgs &p, float *dq_acc) {
  * rows, one head of 1000 rows 24.4 against 27.1.  One wave per SIMD with K and V
  * in registers and three buffers took 97 and 24.4 us (128 heads of 4096 causal:
  * 694 against 522 us).
- * As in attn_bwd_fused, the dP MFMAs run on -V (negated once in LDS) and
+ * As in attn_dkdv_1w, the dP MFMAs run on -V (negated once in LDS) and
  * start from Delta, so they deliver Delta - dP, and the kernel carries
  * -dS = P (Delta - dP) with one multiply; the arithmetic is the same as that
  * kernel's, so dK and dV are bit-identical. */

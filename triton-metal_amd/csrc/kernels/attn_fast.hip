@@ -23,12 +23,21 @@ TM_PRE_FAST(f16_t, f16, 128)
     __shared__ __align__(1024) char lds[Dkdv2wLds<D>::BYTES];                                 \
     attn_dkdv_2w<T, D, CAUSAL>(p, lds, blockIdx.x, gridDim.x);                                \
   }
+#define TM_DKDV_1W(T, TN, CAUSAL, CN)                                                         \
+  extern "C" __global__ __launch_bounds__(256) void tm_attn_dkdv_fast_##TN##_d64##CN##_1w(    \
+      TmAttnDkdvArgs p) {                                                                     \
+    attn_dkdv_1w<T, 64, CAUSAL, false>(p);                                                    \
+  }
+TM_DKDV_1W(bf16_t, bf16, false, )
+TM_DKDV_1W(bf16_t, bf16, true, _causal)
+TM_DKDV_1W(f16_t, f16, false, )
+TM_DKDV_1W(f16_t, f16, true, _causal)
 /* Single-pass backward with atomic dQ (opt-in: bwd=atomic): the dK/dV
  * kernel plus dQ = dS K per query block, and the passes around it. */
 #define TM_BWD_FUSED(T, TN, D, CAUSAL, CN)                                                    \
   extern "C" __global__ __launch_bounds__(256) void tm_attn_fused_fast_##TN##_d##D##CN(       \
       TmAttnFusedArgs p) {                                                                    \
-    attn_bwd_fused<T, D, CAUSAL>(p.kv, p.dq_acc);                                       \
+    attn_dkdv_1w<T, D, CAUSAL, true>(p.kv, p.dq_acc);                                         \
   }
 #define TM_BWD_FAST_ALL(T, TN)           \
   TM_BWD_FUSED(T, TN, 64, false, )       \

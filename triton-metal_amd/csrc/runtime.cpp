@@ -1054,6 +1054,15 @@ int64_t fast_ranges(int64_t wgs, int64_t n_ctx, int head_dim) {
   return std::max<int64_t>(1, std::min<int64_t>({2 * cus / wgs, n_ctx / 256, 16}));
 }
 
+/* Where the head_dim 64 dK/dV runs one wave per SIMD (attn_dkdv_1w): a grid of one
+ * workgroup per compute unit has no second wave to hide the softmax of
+ * attn_dkdv_2w, and past the prologue the wave's own pipeline hides it.  bf16
+ * causal, us, one wave and two: 8 heads of 3000 rows 58.7 and 66.4, 16 of 1100
+ * 27.9 and 29.1; 8 of 500 16.5 and 15.9; 40 of 1100 (360 workgroups) 41.8 and 38.4. */
+bool dkdv_one_wave(const BuiltinSpec &spec, int64_t wgs, int64_t n_ctx) {
+  return spec.head_dim == 64 && n_ctx > 1024 && wgs <= device().compute_units;
+}
+
 /* The split form of a generic dq or dkdv plan: the main dispatch over
  * `splits` ranges (grid z) writing fp32 partials to `part`, then the reduce
  * dispatch that sums them into the outputs (dQ * sm_scale, or dK * sm_scale
@@ -1390,6 +1399,7 @@ Plan plan_builtin(Kernel &k, const Library &lib, const std::vector<Arg> &args, i
           plan_split_backward(plan, spec, p, (float *)work, splits, fast, p.dk, p.dv);
           return plan;
         }
+        if (fast && !width && dkdv_one_wave(spec, plan.grid[0], n_ctx)) plan.variant += "_1w";
         set_kernarg(plan, p);
       }
       break;
