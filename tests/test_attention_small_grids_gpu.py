@@ -1,7 +1,12 @@
-"""The forms that small grids keep: the head_dim 64 dK/dV with one wave per SIMD, against the fp64 oracle."""
+"""The forms that small grids keep: the head_dim 64 dK/dV with one wave per SIMD and
+the fp32 forward on the fp32 MFMAs at 65 to 80 columns, against the fp64 oracle."""
+
+import math
 
 import pytest
 
+from oracle import reference as R
+from oracle import tolerance as T
 from test_fast_paths_gpu import _attention, _check
 from triton_metal import _core, ops
 
@@ -30,3 +35,16 @@ def test_short_walks_and_larger_grids_take_two_waves(device, heads, seq):
         assert _core.kernel_variant(layer.lib.kernels["attn_bwd_dkdv"]) == "tm_attn_dkdv_fast_bf16_d64"
     finally:
         layer.free()
+
+
+@pytest.mark.parametrize("causal", [False, True])
+@pytest.mark.parametrize("heads,seq,dim,pad,kept", [
+    (2, 1, 80, 0, True), (3, 65, 65, 1, True), (6, 113, 80, 3, True), (2, 512, 72, 0, True),
+    (2, 513, 80, 0, False), (2, 100, 81, 0, False), (65, 128, 80, 0, False),
+])
+def test_fp32_forward_65_to_80(device, heads, seq, dim, pad, causal, kept):
+    out, variants, dense, _ = _attention(heads, seq, dim, "f32", causal, stride_seq=dim + pad)
+    assert ("_mfma32" in variants[0]) == kept, variants
+    want = R.attention_backward(*dense, 1 / math.sqrt(dim), causal)
+    assert T.hybrid_error(out["o"], want["o"]) <= 2e-5
+    assert T.hybrid_error(out["lse"], want["lse"]) <= 2e-5

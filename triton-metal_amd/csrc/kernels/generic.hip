@@ -1,11 +1,13 @@
 /*
- * Generic gfx950 kernels for the dense hot path: every element type the
- * reference supports (f32, f16, bf16), arbitrary strides, ragged shapes, any
- * head dimension up to 128, causal or not.  They stage tiles through LDS as
- * f32 and contract on v_mfma_f32_16x16x4_f32, which multiplies exactly for all
- * three element types, so one code path serves them all.  The hot shapes run
- * on the specialised kernels in gemm_fast.hip / attn_fast.hip; these cover
- * everything else with the reference's numerics:
+ * Generic gfx950 kernels for the dense hot path: arbitrary strides, ragged
+ * shapes, any head dimension up to 128, causal or not.  They stage tiles through
+ * LDS as f32 and contract on v_mfma_f32_16x16x4_f32, which multiplies exactly
+ * for all three element types (gemm_generic.h, attn_generic.h).  What runs here:
+ * 16-bit attention whose rows are not 16-byte aligned, whose head dimension is
+ * no multiple of 8, or whose grid is tiny (ranges fill the chip); fp32 products
+ * of at most 32 columns of K or of strides that are not 1; the range combines
+ * and reduces; Delta.  (fp32 attention: attn_x3.hip, with these bodies as its
+ * fallback.)  The reference's numerics:
  *   - f32 accumulation everywhere (GEMMKernel.swift:46, AttentionKernel.swift:59-65);
  *   - P and dS rounded to the element type before the dot they feed
  *     (AttentionKernel.swift:59-65, AttentionBackwardKernel.swift:155-160, :357-369);
@@ -186,6 +188,17 @@ TM_SPLIT_REDUCE(bf16_t, bf16)
 TM_PRE(float, tm_attn_pre_generic_f32)
 TM_PRE(f16_t, tm_attn_pre_generic_f16)
 TM_PRE(bf16_t, tm_attn_pre_generic_bf16)
+
+/* the fp32 forward on the fp32 MFMAs, beside attn_x3.hip's (65 to 80 columns, short
+ * sequences of few heads) */
+#define TM_FWD_F32(DP, CAUSAL, CN)                                                            \
+  extern "C" __global__ __launch_bounds__(256) void tm_attn_fwd_generic_f32_d##DP##CN##_mfma32( \
+      TmAttnFwdArgs p) {                                                                      \
+    __shared__ __align__(16) float k[generic_tile(DP)], v[generic_tile(DP)];                  \
+    attn_fwd_generic<float, DP, CAUSAL>(p, k, v);                                             \
+  }
+TM_FWD_F32(96, false, )
+TM_FWD_F32(96, true, _causal)
 
 #define TM_ATTN_ONE(T, TN, DP, CAUSAL, CN)                                                    \
   extern "C" __global__ __launch_bounds__(256) void tm_attn_fwd_generic_##TN##_d##DP##CN(     \

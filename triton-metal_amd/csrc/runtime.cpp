@@ -1054,6 +1054,17 @@ int64_t fast_ranges(int64_t wgs, int64_t n_ctx, int head_dim) {
   return std::max<int64_t>(1, std::min<int64_t>({2 * cus / wgs, n_ctx / 256, 16}));
 }
 
+/* Where the fp32 forward keeps the fp32 MFMAs: at 65 to 80 columns the split form
+ * contracts 96, which costs more than the faster MFMAs save while a grid leaves
+ * half the compute units idle (`wgs` workgroups of 64 queries) and walks at most
+ * 512 keys.  us, fp32 MFMA and split, 80 columns: 6 heads of 113 rows 14.7 and
+ * 15.7, 16 of 256 19.1 and 20.1, 4 of 512 17.9 and 19.1; 40 of 300 49.7 and 47.1;
+ * 4 of 600 28.5 and 26.8; 96 columns, 16 of 256 20.5 and 19.0. */
+bool fwd_fp32_mfma(const BuiltinSpec &spec, int64_t wgs, int64_t n_ctx) {
+  return spec.element == Element::F32 && spec.head_dim > 64 && spec.head_dim <= 80 &&
+         n_ctx <= 512 && 2 * wgs <= device().compute_units;
+}
+
 /* Where the head_dim 64 dK/dV runs one wave per SIMD (attn_dkdv_1w): a grid of one
  * workgroup per compute unit has no second wave to hide the softmax of
  * attn_dkdv_2w, and past the prologue the wave's own pipeline hides it.  bf16
@@ -1231,6 +1242,7 @@ Plan plan_builtin(Kernel &k, const Library &lib, const std::vector<Arg> &args, i
         plan.variant = attn_symbol("fwd", spec);
         plan.grid[0] = (unsigned)cdiv(p.n_ctx, 64);
         plan.grid[1] = (unsigned)heads;
+        if (fwd_fp32_mfma(spec, (int64_t)plan.grid[0] * heads, p.n_ctx)) plan.variant += "_mfma32";
         plan.block = 256;
         /* Too few 64-query workgroups to fill the chip twice, each walking
          * many key blocks: split every workgroup's key blocks into `splits`
