@@ -12,7 +12,7 @@
  * workgroup per CU; each wave owns a 128 x 128 sub-tile as 4 x 4
  * accumulators of v_mfma_f32_32x32x16_{bf16,f16} (256 accumulator registers:
  * the kernel is built for one wave per SIMD and 512 registers).  Against the
- * 8-wave kernel of gemm_fast.hip (128 x 64 per wave, 16x16x32) this reads a
+ * 8-wave kernel of gemm_fast.h (128 x 64 per wave, 16x16x32) this reads a
  * third less LDS per K step (each wave's operands cover twice the columns),
  * and the 32x32x16 instruction issues closer to the MFMA peak.
  *
@@ -28,7 +28,7 @@
  * which hide its LDS latency.  C goes out through LDS in whole row segments.
  *
  * Measured at 8192^3 on one MI355X (alternating runs, TFLOP/s): this kernel
- * 1311-1342 against 1291-1341 for gemm_fast.hip's 8-wave kernel, the SAE
+ * 1311-1342 against 1291-1341 for gemm_fast.h's 8-wave kernel, the SAE
  * encoder shape (8192 x 2048 -> 16384) 1166 against 1080, and short K
  * (4096^2 x 64 / 128) 11.6 / 12.7 us against 14.1 / 15.3; B transposed
  * 1315-1321 against 1289-1298, A transposed 1297-1304 against 1218-1222.
@@ -43,7 +43,7 @@
  * gives a fragment by one ds_read_b128; the other kind a [64][256] tile of
  * 512-byte rows and two ds_read_b64_tr_b16 (W4Operand).  The product is then
  * C^T: a lane holds 4 consecutive columns of one row per group of 4
- * accumulator floats.  Tiles keep gemm_fast.hip's layouts with XOR keys for
+ * accumulator floats.  Tiles keep gemm_fast.h's layouts with XOR keys for
  * this kernel's 32-row reads.
  */
 #include "common.h"
@@ -74,13 +74,13 @@ TM_DEV int w4_xcd_remap(int wg, int nwg) {
  * c ^ ((r >> 1) & 7).  A ds_read_b128 of 32 lanes reads 32 consecutive rows
  * at one chunk: two rows share each 256-byte bank line, so the row's parity
  * and the key give 16 distinct 16-byte slots (the row & 7 key of
- * gemm_fast.hip, made for 16 rows, gives 8 here: 2-way conflicts). */
+ * gemm_fast.h, made for 16 rows, gives 8 here: 2-way conflicts). */
 TM_DEV int w4_a_swz(int row) { return (row >> 1) & 7; }
 TM_DEV int w4_a_off(int row, int chunk) { return row * 128 + ((chunk ^ w4_a_swz(row)) << 4); }
 /* B tile [64 k][256 n], 512-byte rows.  A transposed read of 32 lanes
  * touches 4 consecutive rows at 4 consecutive chunks (two 16-lane groups
  * side by side); the key 4 (row & 3) puts the 4 rows' chunks in 4 disjoint
- * blocks of the 256-byte bank width.  (gemm_fast.hip's key, made for 8 rows
+ * blocks of the 256-byte bank width.  (gemm_fast.h's key, made for 8 rows
  * at one chunk pair, leaves these reads 2-way conflicted.) */
 TM_DEV int w4_b_swz(int row) { return (row & 3) << 2; }
 TM_DEV int w4_b_off(int row, int chunk) { return row * 512 + ((chunk ^ w4_b_swz(row)) << 4); }
