@@ -61,3 +61,21 @@ def test_sae_k_groups(device, rows, model, features, kernel):
     variant = _core.kernel_variant(enc.kernel)
     assert T.hybrid_error(got, R.sae_encode(x, w, b)) <= 2e-2, variant
     assert variant == f"tm_sae_{kernel}_bf16"
+
+
+@pytest.mark.parametrize("element", ["bf16", "f16"])
+@pytest.mark.parametrize("layout", ["nn", "nt", "tn"])
+@pytest.mark.parametrize("m,n,k", [(16, 20000, 1024), (63, 16460, 901)])
+def test_k_ranges_of_more_tiles_than_compute_units(device, element, layout, m, n, k):
+    up = lambda x: -(-(x + 1) // 8) * 8
+    if layout == "nn":
+        c, want, got = _gemm(m, n, k, element, up(k), up(n), up(n), poison=True, extra_rows=3)
+    elif layout == "nt":
+        c, want, got = _gemm_nt(m, n, k, element, up(k), up(k), up(n))
+    else:
+        c, want, got = _gemm_tn(m, n, k, element, up(m), up(n), up(n))
+    suffix = "" if layout == "nn" else "_" + layout
+    assert got.split(" + ")[0] == f"tm_gemm_ragged{suffix}_t64_ks_{element}"
+    assert np.all(np.isfinite(c[:m, :n]))
+    assert T.hybrid_error(c[:m, :n], want) <= 2e-2
+    assert np.all(c[:m, n:] == -7.0) and np.all(c[m:] == -7.0)

@@ -957,6 +957,7 @@ bool plan_gemm_split(Plan &plan, TmGemmArgs &p, const BuiltinSpec &spec, const L
   if (!TM_GEMM_SPLITK || spec.element == Element::F32 || plan.variant.rfind("tm_gemm_", 0) != 0 ||
       (!unaligned && plan.variant.find("_t64") == std::string::npos))
     return false;
+  const bool ragged = plan.variant.find("ragged") != std::string::npos;
   const int64_t cus = std::max(device().compute_units, 1);
   const int64_t tiles = plan.grid[0];
   const int64_t kg = plan.block / 128; /* wave groups of the K split inside the workgroup */
@@ -969,19 +970,18 @@ bool plan_gemm_split(Plan &plan, TmGemmArgs &p, const BuiltinSpec &spec, const L
    * 512 x 512 x 3072, which saves 9, 10.5 split); of two ranges, half the
    * partials, as six (200 x 2000 x 3000: 15.0 split, 17.8 not) */
   if (splits < 2 || (ksteps - ksteps / splits) / kg < (splits == 2 ? 6 : 8)) return false;
+  /* one group of whole tiles means more tiles than fill the chip (choose_gemm) */
+  if (!unaligned && !ragged && kg != 4) return false;
   const int64_t np = (p.n + 3) & ~int64_t(3);
   void *work = plan_workspace(lib, (size_t)splits * (size_t)p.m * (size_t)np * 4, scratch);
   if (!work) return false;
   p.part = (float *)work;
   p.splits = (int32_t)splits;
   Plan main = plan, reduce;
-  /* the "_ks" instantiation of the planned kernel */
-  const bool ragged = plan.variant.find("ragged") != std::string::npos;
-  const std::string suffix = std::string("_") + el;
-  main.variant = unaligned ? format("tm_gemm_unaligned%s_t64",
-                                    p.layout == TM_GEMM_NT ? "_nt" : p.layout == TM_GEMM_TN ? "_tn" : "")
-                           : plan.variant.substr(0, plan.variant.size() - suffix.size());
-  main.variant += (unaligned || ragged) && kg == 4 ? "_k4_ks" + suffix : "_ks" + suffix;
+  /* the "_ks" instantiation of the planned kernel's tiles, layout and groups */
+  main.variant = format("tm_gemm_%s%s_t64%s_ks_%s", unaligned ? "unaligned" : ragged ? "ragged" : "fast",
+                        p.layout == TM_GEMM_NT ? "_nt" : p.layout == TM_GEMM_TN ? "_tn" : "",
+                        kg == 4 ? "_k4" : "", el);
   main.lds = 0;
   main.grid[1] = (unsigned)splits;
   set_kernarg(main, p);
