@@ -66,6 +66,18 @@ def test_x3_gemm(device, layout, m, n, k, pad, kernel):
     _check(c, a, b, k)
 
 
+@pytest.mark.parametrize("m,n,k,layout", [(2048, 1088, 8192, "nn"), (1088, 2048, 8192, "tn")])
+def test_x3_operands_of_whole_2_mib(device, m, n, k, layout):
+    """128 x 128 tiles, the last one 64 wide, over an operand that ends where its
+    allocation ends (tests/test_x3_runs.py: no load leaves it)."""
+    rng = np.random.default_rng(4)
+    a = rng.standard_normal((m, k), dtype=np.float32)
+    b = rng.standard_normal((k, n), dtype=np.float32)
+    c, got = _run(a, b, layout, 0)
+    assert got.split(" + ")[0] == f"tm_gemm_x3{'_tn' if layout == 'tn' else ''}_f32"
+    _check(c, a, b, k)
+
+
 @pytest.mark.parametrize("layout", ["nn", "nt", "tn"])
 @pytest.mark.parametrize("scale", [2.0 ** -115, 2.0 ** -99, 2.0 ** 60, 2.0 ** 100])
 def test_x3_keeps_small_and_large_values(device, layout, scale):

@@ -24,6 +24,7 @@
  */
 #include "gemm_fast.h"
 #include "split3.h"
+#include "x3_runs.h"
 
 namespace {
 
@@ -39,11 +40,10 @@ TM_DEV int x3_off(int row, int chunk) { return row * 64 + ((chunk ^ ((row >> 2) 
 /* One operand's tile: TILE x 32 floats through registers, eight per task, into
  * three bf16 planes of TILE * 64 bytes.  CONTIG: k is the contiguous dimension
  * (planes [TILE][32]), else the other one is (planes [32][TILE], gemm_fast.h's
- * B layout).  Loads are 16 bytes at any 4-byte address, up to 12 bytes past the
- * operand.  Rows past the matrix repeat the last one, runs past its last column
- * start at it, and what is then not of the matrix is replaced by zeros: k past K
- * because it would be added, columns so that a stray value does not send the
- * workgroup to its fp32 path. */
+ * B layout).  Loads are 16 bytes at any 4-byte address, where x3_runs.h says.
+ * What is then not of the matrix is replaced by zeros: k past K because it would
+ * be added, columns so that a stray value does not send the workgroup to its fp32
+ * path. */
 template <bool CONTIG, int TILE>
 struct X3Tile {
   static constexpr int TASKS = TILE / 64, CPR = CONTIG ? 4 : TILE / 8, RPT = 256 / CPR;
@@ -60,9 +60,7 @@ struct X3Tile {
     for (int t = 0; t < TASKS; ++t)
 #pragma unroll
       for (int h = 0; h < 2; ++h) {
-        const int row = row0 + t * RPT, col = chunk * 8 + h * 4;
-        off[t][h] = 4 * (CONTIG ? (uint32_t)(min(row, rows - 1) * ld) + col
-                                : (uint32_t)(row * ld) + min(col, rows - 1));
+        off[t][h] = x3_run<CONTIG>(ld, row0 + t * RPT, chunk * 8 + h * 4, rows);
       }
   }
   TM_DEV void load(const float *base, int64_t ld, int k_left) {
@@ -77,17 +75,10 @@ struct X3Tile {
       for (int t = 0; t < TASKS; ++t)
 #pragma unroll
         for (int h = 0; h < 2; ++h) {
-          if (CONTIG) {
-            const int col = chunk * 8 + h * 4;
-            const f32x4 x = *(const f32x4_any *)(src + (off[t][h] - 4 * max(col - (k_left - 1), 0)));
+          const int row = row0 + t * RPT, col = chunk * 8 + h * 4;
+          const f32x4 x = *(const f32x4_any *)(src + x3_last_run<CONTIG>(off[t][h], ld, row, col, k_left));
 #pragma unroll
-            for (int e = 0; e < 4; ++e) v[t][h][e] = col + e < k_left ? x[e] : 0.f;
-          } else {
-            const int row = row0 + t * RPT;
-            const bool in = row < k_left;
-            const f32x4 x = *(const f32x4_any *)(src + (in ? off[t][h] : off[t][h] - 4 * (uint32_t)(row * ld)));
-            v[t][h] = in ? x : (f32x4){0.f, 0.f, 0.f, 0.f};
-          }
+          for (int e = 0; e < 4; ++e) v[t][h][e] = (CONTIG ? col + e : row) < k_left ? x[e] : 0.f;
         }
     }
     if (!CONTIG && width < TILE) {

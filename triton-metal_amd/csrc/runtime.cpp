@@ -734,8 +734,9 @@ void choose_gemm(Plan &plan, TmGemmArgs &p, const BuiltinSpec &spec, const char 
     const bool b_t = gemm && !b_n && p.sbk == 1 && p.sbn % 4 == 0 && p.sbn >= p.k;
     const int tile = f32_big ? 128 : 64;
     const int64_t tiles = (int64_t)(p.m / tile) * (p.n / tile);
-    /* the bf16-split kernel (whole tiles of 16-byte aligned rows leave it nothing
-     * to read past an operand), us against this one's: more 128 x 128 tiles than
+    /* the bf16-split kernel (M, N and K of whole 16-byte runs leave it nothing to
+     * read past an operand, whichever tile it takes: x3_runs.h), us against this
+     * one's: more 128 x 128 tiles than
      * compute units 725 / 1050 (4096^3); up to as many, past K = 1024, 109 / 134
      * (2048 x 2048 x 1984), 64 / 135 (2048 x 1024 x 2016, B transposed); 64 x 64
      * tiles for half the compute units, from K = 512 in ranges, 16 / 23 (512 x
