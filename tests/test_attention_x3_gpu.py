@@ -79,3 +79,37 @@ def test_infinities_stay_in_their_columns(device):
     keep[3] = False
     assert T.hybrid_error(got["o"][0][:, keep], want[0][:, keep]) <= 2e-5
     assert T.hybrid_error(got["o"][1], want[1]) <= 2e-5
+
+
+def test_small_probabilities_and_score_gradients(device):
+    """P and dS near the bottom of the range from operands that are not: their
+    parts keep fp32's bits."""
+    x = _inputs()
+    scale = 1 / 8.0
+    want = R.attention_backward(x["q"], x["k"], x["v"], x["do"], scale, False)
+    x["v"], x["do"] = np.ldexp(x["v"], -24), np.ldexp(x["do"], -96)
+    got = _layer(x, scale)
+    for out, power in {"o": -24, "dq": -120, "dk": -120, "dv": -96}.items():
+        assert T.hybrid_error(np.ldexp(got[out].astype(np.float64), -power), want[out]) <= 1e-4, out
+
+    x = _inputs()
+    x["q"][:, :, 0] = 8.0
+    x["k"][:, :, 0] = 0.0
+    x["k"][:, 0] = 0.0
+    x["k"][:, 0, 0] = -83.2  # key 0: P of about 2^-125 for every query
+    got = _layer(x, scale)
+    want = R.attention_backward(x["q"], x["k"], x["v"], x["do"], scale, False)
+    small, exact = got["dv"][:, 0].astype(np.float64), want["dv"][:, 0]
+    assert np.linalg.norm(exact) < 2.0 ** -105
+    assert np.linalg.norm(small - exact) <= 1e-4 * np.linalg.norm(exact)
+
+
+@pytest.mark.parametrize("sign", [1.0, -1.0])
+def test_scores_past_the_scaled_range(device, sign):
+    """Scores of 2^100 and a scale that brings them back: the fp32 body."""
+    x = _inputs(seq=100)
+    want = R.attention_backward(x["q"], x["k"], x["v"], x["do"], sign / 8.0, True)
+    x["q"], x["k"] = np.ldexp(x["q"], 50), np.ldexp(x["k"], 50)
+    got = _layer(x, sign * 2.0 ** -103, causal=True)
+    for out, power in {"o": 0, "lse": 0, "dq": -50, "dk": -50, "dv": 0}.items():
+        assert T.hybrid_error(np.ldexp(got[out].astype(np.float64), -power), want[out]) <= 1e-4, out

@@ -143,3 +143,31 @@ def test_x3_sae(device, rows, model, features):
     want = R.sae_encode(x, w, b)
     bound = (model + 1) * 2.0 ** -24 * (np.abs(x).astype(np.float64) @ np.abs(w) + np.abs(b))
     assert np.all(np.abs(got - want) <= bound)
+
+
+@pytest.mark.parametrize("layout", ["nn", "nt", "tn"])
+def test_x3_keeps_subnormal_values_and_results(device, layout):
+    """Every fp32 number is split without loss, beside ordinary ones; results are
+    rounded once more where fp32 itself is short of bits."""
+    rng = np.random.default_rng(3)
+    m, n, k = 70, 90, 77
+    a = rng.standard_normal((m, k)).astype(np.float32)
+    b = rng.standard_normal((k, n)).astype(np.float32)
+    a[:20] = np.ldexp(a[:20], -135)
+    b[:, :30] = np.ldexp(b[:, :30], 100)
+    c, got = _run(a, b, layout, 1)
+    assert "_x3" in got
+    _check(c, a, b, k)
+
+
+@pytest.mark.parametrize("power", [40, 55])
+def test_x3_results_past_the_scaled_range(device, power):
+    """Results from 2^96 on are computed in fp32."""
+    rng = np.random.default_rng(4)
+    m, n, k = 140, 130, 65
+    a = np.ldexp(rng.standard_normal((m, k)), power).astype(np.float32)
+    b = np.ldexp(rng.standard_normal((k, n)), power).astype(np.float32)
+    b[:, 64:] = np.ldexp(b[:, 64:], -power)
+    c, got = _run(a, b, "nn", 1)
+    assert "_x3" in got
+    _check(c, a, b, k)

@@ -49,13 +49,10 @@ TM_DEV void load8(const float *row, int d, int D, bool in, f32x4 (&v)[2]) {
   }
 }
 
-TM_DEV void split_run(const f32x4 (&v)[2], u32x4 (&part)[3], uint32_t &least) {
+TM_DEV void split_run(const f32x4 (&v)[2], u32x4 (&part)[3]) {
   float x[8];
 #pragma unroll
-  for (int e = 0; e < 8; ++e) {
-    x[e] = v[e >> 2][e & 3];
-    least = x3_least(least, x[e]);
-  }
+  for (int e = 0; e < 8; ++e) x[e] = v[e >> 2][e & 3] * X3_SCALE;
   x3_split8(x, part);
 }
 
@@ -72,13 +69,13 @@ struct Rows {
       load8(base + (int64_t)row * ss, (i % CPR) * 8, D, i < R * CPR && row < n, v[t]);
     }
   }
-  TM_DEV void store(char *lds, int tid, uint32_t &least) const {
+  TM_DEV void store(char *lds, int tid) const {
 #pragma unroll
     for (int t = 0; t < TASKS; ++t) {
       const int i = tid + t * 256;
       if (R * CPR % 256 && i >= R * CPR) break;
       u32x4 part[3];
-      split_run(v[t], part, least);
+      split_run(v[t], part);
       const int at = tile_off<P>(i / CPR, i % CPR);
 #pragma unroll
       for (int q = 0; q < 3; ++q) *(u32x4 *)(lds + q * (R * P * 2) + at) = part[q];
@@ -88,12 +85,12 @@ struct Rows {
 
 /* this lane's row (query or key) as a split MFMA operand, per 32 columns */
 template <int DP>
-TM_DEV void own_row(const float *row, bool in, int D, int g, u32x4 (&part)[DP / 32][3], uint32_t &least) {
+TM_DEV void own_row(const float *row, bool in, int D, int g, u32x4 (&part)[DP / 32][3]) {
 #pragma unroll
   for (int ks = 0; ks < DP / 32; ++ks) {
     f32x4 v[2];
     load8(row, ks * 32 + 8 * g, D, in, v);
-    split_run(v, part[ks], least);
+    split_run(v, part[ks]);
   }
 }
 
@@ -112,12 +109,21 @@ TM_DEV void k_operand(uint32_t tile, uint32_t off, int r0, u32x4 (&part)[3]) {
   for (int q = 0; q < 3; ++q)
     part[q] = lds_read_kmajor(tile + off, q * PLANE + r0 * P * 2, q * PLANE + (r0 + 16) * P * 2);
 }
-/* eight fp32 results of two 16-row tiles (rows 4g + r of each) as the other
- * operand of a k-major product */
-TM_DEV void result_operand(const f32x4 &a, const f32x4 &b, u32x4 (&part)[3]) {
-  float x[8] = {a[0], a[1], a[2], a[3], b[0], b[1], b[2], b[3]};
+/* eight fp32 results of two 16-row tiles (rows 4g + r of each), `scale` times as
+ * large, as the other operand of a k-major product */
+TM_DEV void result_operand(const f32x4 &a, const f32x4 &b, float scale, u32x4 (&part)[3]) {
+  float x[8] = {a[0] * scale, a[1] * scale, a[2] * scale, a[3] * scale,
+                b[0] * scale, b[1] * scale, b[2] * scale, b[3] * scale};
   x3_split8(x, part);
 }
+
+/* what a product of two (three) split operands comes out as, undone */
+constexpr float SCALE2 = X3_SCALE * X3_SCALE, UNSCALE2 = 1.f / SCALE2, UNSCALE3 = UNSCALE2 / X3_SCALE;
+/* (a score scale below this would be rounded when UNSCALE2 is folded into it) */
+TM_DEV bool scale_beyond(float qk_scale) { return fabsf(qk_scale) < 0x1p-90f; }
+/* scores past the range, which the exponential would take to an ordinary 0: the
+ * sum of 0 s is not 0 */
+TM_DEV void note_finite(float &sum, float s) { sum = __builtin_fmaf(s, 0.f, sum); }
 
 /* lane parts of the operand addresses */
 template <int DP>
@@ -144,11 +150,10 @@ TM_DEV void attn_fwd_x3(const TmAttnFwdArgs &p, char *lds) {
   const int64_t base = (int64_t)bh * p.stride_head, ss = p.stride_seq;
   const float *Q = (const float *)p.q + base, *K = (const float *)p.k + base, *V = (const float *)p.v + base;
   const int qi = q0 + wave * 16 + c;
-  uint32_t least = X3_NONE;
   u32x4 qf[KS][3];
-  own_row<DP>(Q + (int64_t)qi * ss, qi < n, D, g, qf, least);
+  own_row<DP>(Q + (int64_t)qi * ss, qi < n, D, g, qf);
   const Lane<DP> at(g, c);
-  const float qk_scale = p.sm_scale * TM_LOG2E;
+  const float qk_scale = p.sm_scale * TM_LOG2E, s_scale = qk_scale * UNSCALE2;
   float m_i = TM_NEG_INF, l_i = 0.f;
   f32x4 acc[DT];
 #pragma unroll
@@ -164,11 +169,11 @@ TM_DEV void attn_fwd_x3(const TmAttnFwdArgs &p, char *lds) {
     kr.load(K, kbeg, n, D, ss, tid);
     vr.load(V, kbeg, n, D, ss, tid);
   }
-  bool beyond = false;
+  float seen = 0.f;
   for (int k0 = kbeg; k0 < kend; k0 += BN) {
     __syncthreads();
-    kr.store(lds, tid, least);
-    vr.store(lds + planes(DP), tid, least);
+    kr.store(lds, tid);
+    vr.store(lds + planes(DP), tid);
     __syncthreads();
     if (k0 + BN < kend) {
       kr.load(K, k0 + BN, n, D, ss, tid);
@@ -192,8 +197,8 @@ TM_DEV void attn_fwd_x3(const TmAttnFwdArgs &p, char *lds) {
 #pragma unroll
       for (int r = 0; r < 4; ++r) {
         const int kj = k0 + kt * 16 + 4 * g + r;
-        beyond |= x3_not_finite(s[kt][r]);
-        float v = s[kt][r] * qk_scale;
+        note_finite(seen, s[kt][r]);
+        float v = s[kt][r] * s_scale;
         if (kj >= n || (CAUSAL && kj > qi)) v = TM_NEG_INF;
         s[kt][r] = v;
         mx = fmaxf(mx, v);
@@ -218,7 +223,7 @@ TM_DEV void attn_fwd_x3(const TmAttnFwdArgs &p, char *lds) {
 #pragma unroll
     for (int kk = 0; kk < BN / 32; ++kk) {
       u32x4 pf[3];
-      result_operand(s[2 * kk], s[2 * kk + 1], pf);
+      result_operand(s[2 * kk], s[2 * kk + 1], X3_SCALE, pf);
 #pragma unroll
       for (int dt = 0; dt < DT; dt += 2) {
         u32x4 a[3], b[3];
@@ -228,7 +233,7 @@ TM_DEV void attn_fwd_x3(const TmAttnFwdArgs &p, char *lds) {
       }
     }
   }
-  beyond |= x3_below(least);
+  bool beyond = scale_beyond(qk_scale) || seen != 0.f;
 #pragma unroll
   for (int dt = 0; dt < DT; ++dt)
 #pragma unroll
@@ -244,7 +249,7 @@ TM_DEV void attn_fwd_x3(const TmAttnFwdArgs &p, char *lds) {
 #pragma unroll
       for (int r = 0; r < 4; ++r) {
         const int d = dt * 16 + 4 * g + r;
-        if (d < D) po[d] = acc[dt][r];
+        if (d < D) po[d] = acc[dt][r] * UNSCALE2;
       }
     if (g == 0) {
       float *pml = p.part + (int64_t)p.splits * p.heads * n * D + (((int64_t)split * p.heads + bh) * n + qi) * 2;
@@ -253,7 +258,7 @@ TM_DEV void attn_fwd_x3(const TmAttnFwdArgs &p, char *lds) {
     }
   } else if (qi < n) {
     float *O = (float *)p.o + base + (int64_t)qi * ss;
-    const float inv = 1.f / l_i;
+    const float inv = 1.f / l_i * UNSCALE2;
 #pragma unroll
     for (int dt = 0; dt < DT; ++dt)
 #pragma unroll
@@ -277,15 +282,15 @@ TM_DEV void attn_dq_x3(const TmAttnDqArgs &p, char *lds) {
   const int64_t base = (int64_t)bh * p.stride_head, ss = p.stride_seq;
   const float *K = (const float *)p.k + base, *V = (const float *)p.v + base;
   const int qi = q0 + wave * 16 + c;
-  uint32_t least = X3_NONE;
   u32x4 qf[KS][3], df[KS][3];
-  own_row<DP>((const float *)p.q + base + (int64_t)qi * ss, qi < n, D, g, qf, least);
-  own_row<DP>((const float *)p.dout + base + (int64_t)qi * ss, qi < n, D, g, df, least);
+  own_row<DP>((const float *)p.q + base + (int64_t)qi * ss, qi < n, D, g, qf);
+  own_row<DP>((const float *)p.dout + base + (int64_t)qi * ss, qi < n, D, g, df);
   const Lane<DP> at(g, c);
   const int64_t srow = (int64_t)bh * p.stride_lse + qi;
   const float lse = qi < n ? p.lse[srow] : 0.f;
-  const float delta = qi < n ? p.delta[srow] : 0.f;
-  const float qk_scale = p.sm_scale * TM_LOG2E;
+  const float delta = qi < n ? p.delta[srow] * SCALE2 : 0.f; /* at dP's scale */
+  const float qk_scale = p.sm_scale * TM_LOG2E, s_scale = qk_scale * UNSCALE2;
+  float seen = 0.f;
   f32x4 acc[DT];
 #pragma unroll
   for (int dt = 0; dt < DT; ++dt) acc[dt] = (f32x4){0.f, 0.f, 0.f, 0.f};
@@ -304,8 +309,8 @@ TM_DEV void attn_dq_x3(const TmAttnDqArgs &p, char *lds) {
   }
   for (int k0 = kbeg; k0 < kend; k0 += BN) {
     __syncthreads();
-    kr.store(lds, tid, least);
-    vr.store(lds + planes(DP), tid, least);
+    kr.store(lds, tid);
+    vr.store(lds + planes(DP), tid);
     __syncthreads();
     if (k0 + BN < kend) {
       kr.load(K, k0 + BN, n, D, ss, tid);
@@ -330,12 +335,13 @@ TM_DEV void attn_dq_x3(const TmAttnDqArgs &p, char *lds) {
 #pragma unroll
         for (int r = 0; r < 4; ++r) {
           const int kj = k0 + kk * 32 + t * 16 + 4 * g + r;
-          float v = s[t][r] * qk_scale;
+          note_finite(seen, s[t][r]);
+          float v = s[t][r] * s_scale;
           if (kj >= n || (CAUSAL && kj > qi)) v = TM_NEG_INF;
           s[t][r] = exp2f(v - lse) * (dp[t][r] - delta);
         }
       u32x4 dsf[3];
-      result_operand(s[0], s[1], dsf);
+      result_operand(s[0], s[1], 1.f, dsf);
 #pragma unroll
       for (int dt = 0; dt < DT; dt += 2) {
         u32x4 a[3], b[3];
@@ -345,7 +351,7 @@ TM_DEV void attn_dq_x3(const TmAttnDqArgs &p, char *lds) {
       }
     }
   }
-  bool beyond = x3_below(least);
+  bool beyond = scale_beyond(qk_scale) || seen != 0.f;
 #pragma unroll
   for (int dt = 0; dt < DT; ++dt)
 #pragma unroll
@@ -363,8 +369,9 @@ TM_DEV void attn_dq_x3(const TmAttnDqArgs &p, char *lds) {
       for (int r = 0; r < 4; ++r) {
         const int d = dt * 16 + 4 * g + r;
         if (d >= D) continue;
-        if (po) po[d] = acc[dt][r];
-        else dq[d] = acc[dt][r] * p.sm_scale;
+        const float x = acc[dt][r] * UNSCALE3;
+        if (po) po[d] = x;
+        else dq[d] = x * p.sm_scale;
       }
   }
 }
@@ -382,12 +389,12 @@ TM_DEV void attn_dkdv_x3(const TmAttnDkdvArgs &p, char *lds, float *Ls, float *D
   const float *Q = (const float *)p.q + base, *dO = (const float *)p.dout + base;
   const float *Lrow = p.lse + (int64_t)bh * p.stride_lse, *Drow = p.delta + (int64_t)bh * p.stride_lse;
   const int kj = k0 + wave * 16 + c;
-  uint32_t least = X3_NONE;
   u32x4 kf[KS][3], vf[KS][3];
-  own_row<DP>((const float *)p.k + base + (int64_t)kj * ss, kj < n, D, g, kf, least);
-  own_row<DP>((const float *)p.v + base + (int64_t)kj * ss, kj < n, D, g, vf, least);
+  own_row<DP>((const float *)p.k + base + (int64_t)kj * ss, kj < n, D, g, kf);
+  own_row<DP>((const float *)p.v + base + (int64_t)kj * ss, kj < n, D, g, vf);
   const Lane<DP> at(g, c);
-  const float qk_scale = p.sm_scale * TM_LOG2E;
+  const float qk_scale = p.sm_scale * TM_LOG2E, s_scale = qk_scale * UNSCALE2;
+  float seen = 0.f;
   f32x4 dk[DT], dv[DT];
 #pragma unroll
   for (int dt = 0; dt < DT; ++dt) dk[dt] = dv[dt] = (f32x4){0.f, 0.f, 0.f, 0.f};
@@ -405,13 +412,13 @@ TM_DEV void attn_dkdv_x3(const TmAttnDkdvArgs &p, char *lds, float *Ls, float *D
     dor.load(dO, q0, n, D, ss, tid);
     const int qi = q0 + tid;
     l_next = tid < BM && qi < n ? Lrow[qi] : 0.f;
-    d_next = tid < BM && qi < n ? Drow[qi] : 0.f;
+    d_next = tid < BM && qi < n ? Drow[qi] * SCALE2 : 0.f; /* at dP's scale */
   };
   if (qstart < qstop) load(qstart);
   for (int q0 = qstart; q0 < qstop; q0 += BM) {
     __syncthreads();
-    qr.store(lds, tid, least);
-    dor.store(lds + planes(DP), tid, least);
+    qr.store(lds, tid);
+    dor.store(lds + planes(DP), tid);
     if (tid < BM) {
       Ls[tid] = l_next;
       Ds[tid] = d_next;
@@ -437,14 +444,15 @@ TM_DEV void attn_dkdv_x3(const TmAttnDkdvArgs &p, char *lds, float *Ls, float *D
 #pragma unroll
         for (int r = 0; r < 4; ++r) {
           const int row = kk * 32 + t * 16 + 4 * g + r, qi = q0 + row;
-          float v = s[t][r] * qk_scale;
+          note_finite(seen, s[t][r]);
+          float v = s[t][r] * s_scale;
           if (qi >= n || (CAUSAL && qi < kj)) v = TM_NEG_INF;
           s[t][r] = exp2f(v - Ls[row]);
           dp[t][r] = s[t][r] * (dp[t][r] - Ds[row]);
         }
       u32x4 pf[3], dsf[3];
-      result_operand(s[0], s[1], pf);
-      result_operand(dp[0], dp[1], dsf);
+      result_operand(s[0], s[1], X3_SCALE, pf);
+      result_operand(dp[0], dp[1], 1.f, dsf);
 #pragma unroll
       for (int dt = 0; dt < DT; ++dt) {
         u32x4 a[3], b[3];
@@ -454,7 +462,7 @@ TM_DEV void attn_dkdv_x3(const TmAttnDkdvArgs &p, char *lds, float *Ls, float *D
       }
     }
   }
-  bool beyond = x3_below(least);
+  bool beyond = scale_beyond(qk_scale) || seen != 0.f;
 #pragma unroll
   for (int dt = 0; dt < DT; ++dt)
 #pragma unroll
@@ -473,12 +481,13 @@ TM_DEV void attn_dkdv_x3(const TmAttnDkdvArgs &p, char *lds, float *Ls, float *D
       for (int r = 0; r < 4; ++r) {
         const int d = dt * 16 + 4 * g + r;
         if (d >= D) continue;
+        const float k = dk[dt][r] * UNSCALE3, v = dv[dt][r] * UNSCALE2;
         if (pk) {
-          pk[d] = dk[dt][r];
-          pk[plane + d] = dv[dt][r];
+          pk[d] = k;
+          pk[plane + d] = v;
         } else {
-          dK[d] = dk[dt][r] * p.sm_scale;
-          dV[d] = dv[dt][r];
+          dK[d] = k * p.sm_scale;
+          dV[d] = v;
         }
       }
   }

@@ -11,16 +11,15 @@
  * Measured (us, fp32 MFMA kernels before and now): 2049 x 3079 x 1025 177 and
  * 94, 4096^3 1050 and 725 (190 TFLOP/s), 1500^3 114 and 61, 1000^3 40 and 28,
  * 129 x 202 x 7481 276 and 27.  At 4096^3 the MFMAs take 55% of the time; the rest
- * is what two workgroups per CU leave uncovered of the split (7 VALU operations
+ * is what two workgroups per CU leave uncovered of the split (6 VALU operations
  * an element), the LDS writes and transposed reads between its barriers.
  * Splitting into registers behind the MFMAs instead ran 93 / 738 us, three
  * workgroups per CU (168 registers) 114 / 818.
  *
- * What the split cannot represent goes back to fp32: values whose hi part
- * overflows, infinities and NaN leave a non-finite accumulator, and values
- * below 2^-100 (whose lo part would be subnormal in bf16) are counted while
- * they are split; a workgroup that meets either computes its tile again on
- * v_mfma_f32_16x16x4_f32, straight from memory.
+ * What the split cannot represent goes back to fp32: values and results near the
+ * top of the range (split3.h), infinities and NaN leave a non-finite accumulator; a
+ * workgroup that meets one computes its tile again on v_mfma_f32_16x16x4_f32,
+ * straight from memory.
  */
 #include "gemm_fast.h"
 #include "split3.h"
@@ -92,17 +91,14 @@ struct X3Tile {
     }
   }
   /* split into the planes at `lds` */
-  TM_DEV void store(char *lds, uint32_t &least) {
+  TM_DEV void store(char *lds) {
 #pragma unroll
     for (int t = 0; t < TASKS; ++t) {
       const int row = row0 + t * RPT;
       const int at = CONTIG ? x3_off(row, chunk) : b_off<TILE>(row, chunk);
       float x[8];
 #pragma unroll
-      for (int e = 0; e < 8; ++e) {
-        x[e] = v[t][e >> 2][e & 3];
-        least = x3_least(least, x[e]);
-      }
+      for (int e = 0; e < 8; ++e) x[e] = v[t][e >> 2][e & 3] * X3_SCALE;
       u32x4 part[3];
       x3_split8(x, part);
 #pragma unroll
@@ -162,12 +158,11 @@ TM_DEV void gemm_x3(const TmGemmArgs &p) {
   for (int i = 0; i < NI; ++i)
 #pragma unroll
     for (int j = 0; j < NI; ++j) acc[i][j] = (f32x4){0.f, 0.f, 0.f, 0.f};
-  uint32_t least = X3_NONE;
 
   if (kbeg < kend) load(kbeg);
   for (int kb = kbeg; kb < kend; ++kb) {
-    ta.store(lds_a, least);
-    tb.store(lds_b, least);
+    ta.store(lds_a);
+    tb.store(lds_b);
     __syncthreads();
     if (kb + 1 < kend) load(kb + 1);
     __builtin_amdgcn_sched_barrier(0);
@@ -202,13 +197,16 @@ TM_DEV void gemm_x3(const TmGemmArgs &p) {
     __syncthreads();
   }
 
-  bool beyond = x3_below(least);
+  bool beyond = false;
 #pragma unroll
   for (int i = 0; i < NI; ++i)
 #pragma unroll
     for (int j = 0; j < NI; ++j)
 #pragma unroll
-      for (int r = 0; r < 4; ++r) beyond |= x3_not_finite(acc[i][j][r]);
+      for (int r = 0; r < 4; ++r) {
+        beyond |= x3_not_finite(acc[i][j][r]);
+        acc[i][j][r] *= 1.f / (X3_SCALE * X3_SCALE);
+      }
   if (__syncthreads_or(beyond)) {
     const int kstop = min(p.k, kend * XK);
 #pragma unroll

@@ -25,13 +25,13 @@ TM_DEV void x3_split8(float (&x)[8], u32x4 (&part)[3]) {
     for (int e = 0; e < 4; ++e) part[q][e] = x3_part(x[2 * e], x[2 * e + 1]);
 }
 
-/* What the parts cannot represent is computed in fp32 instead: magnitudes below
- * 2^-100 (low parts subnormal in bf16), seen in `least`, the smallest of twice
- * the bits less one (zero wraps to the top); overflow and non-finite values show
- * as a non-finite result. */
-constexpr uint32_t X3_NONE = 0xffffffffu;
-TM_DEV uint32_t x3_least(uint32_t least, float x) { return min(least, (__float_as_uint(x) << 1) - 1u); }
-TM_DEV bool x3_below(uint32_t least) { return least < ((27u << 24) - 1u); }
+/* Values are split 2^16 times as large, so that the lowest bit of every fp32
+ * number, 2^-149, is one of bf16's, 2^-133 (the MFMAs and conversions keep
+ * subnormals); results come out 2^32 (2^48: a product of a product) times as large.
+ * What then leaves fp32's range -- a value from 2^112, a result from 2^96 (2^80) --
+ * shows as a non-finite result, as do infinities and NaN, and is computed in fp32
+ * instead. */
+constexpr float X3_SCALE = 0x1p16f;
 TM_DEV bool x3_not_finite(float x) { return !(x - x == 0.f); }
 
 /* two products side by side: a product's six MFMAs wait for each other */
