@@ -160,14 +160,14 @@ def test_x3_keeps_subnormal_values_and_results(device, layout):
     _check(c, a, b, k)
 
 
-@pytest.mark.parametrize("power", [40, 55])
-def test_x3_results_past_the_scaled_range(device, power):
-    """Results from 2^96 on are computed in fp32."""
+@pytest.mark.parametrize("layout", ["nn", "nt", "tn"])
+@pytest.mark.parametrize("m,n,k,power", [(140, 130, 65, 40), (140, 130, 65, 55), (1409, 1281, 77, 50), (64, 200, 1000, 50)])
+def test_x3_results_past_the_scaled_range(device, layout, m, n, k, power):
+    """Results from 2^96 on are computed in fp32: both tile sizes, K ranges."""
     rng = np.random.default_rng(4)
-    m, n, k = 140, 130, 65
     a = np.ldexp(rng.standard_normal((m, k)), power).astype(np.float32)
     b = np.ldexp(rng.standard_normal((k, n)), power).astype(np.float32)
     b[:, 64:] = np.ldexp(b[:, 64:], -power)
-    c, got = _run(a, b, "nn", 1)
+    c, got = _run(a, b, layout, 1)
     assert "_x3" in got
     _check(c, a, b, k)

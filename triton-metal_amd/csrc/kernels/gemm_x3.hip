@@ -18,8 +18,7 @@
  *
  * What the split cannot represent goes back to fp32: values and results near the
  * top of the range (split3.h), infinities and NaN leave a non-finite accumulator; a
- * workgroup that meets one computes its tile again on v_mfma_f32_16x16x4_f32,
- * straight from memory.
+ * workgroup that meets one computes its tile again on v_mfma_f32_16x16x4_f32.
  */
 #include "gemm_fast.h"
 #include "split3.h"
@@ -104,6 +103,20 @@ struct X3Tile {
 #pragma unroll
       for (int q = 0; q < 3; ++q) *(u32x4 *)(lds + q * PLANE + at) = part[q];
     }
+  }
+  /* unsplit, for the fp32 MFMAs: rows of 36 floats (CONTIG), or of TILE + 16, where
+   * the 64 lanes of a read (16 rows or columns at four k) fall on 64 banks */
+  static constexpr int F32_LD = CONTIG ? XK + 4 : TILE + 16;
+  static_assert((CONTIG ? TILE : XK) * F32_LD * 4 <= 3 * PLANE, "LDS");
+  TM_DEV void store_f32(char *lds) {
+#pragma unroll
+    for (int t = 0; t < TASKS; ++t)
+#pragma unroll
+      for (int h = 0; h < 2; ++h)
+        *(f32x4 *)(lds + ((row0 + t * RPT) * F32_LD + chunk * 8 + h * 4) * 4) = v[t][h];
+  }
+  TM_DEV float read_f32(const char *lds, int row, int k) {
+    return ((const float *)lds)[CONTIG ? row * F32_LD + k : k * F32_LD + row];
   }
 };
 
@@ -208,24 +221,30 @@ TM_DEV void gemm_x3(const TmGemmArgs &p) {
         acc[i][j][r] *= 1.f / (X3_SCALE * X3_SCALE);
       }
   if (__syncthreads_or(beyond)) {
-    const int kstop = min(p.k, kend * XK);
 #pragma unroll
     for (int i = 0; i < NI; ++i)
 #pragma unroll
       for (int j = 0; j < NI; ++j) acc[i][j] = (f32x4){0.f, 0.f, 0.f, 0.f};
-    for (int k0 = kbeg * XK; k0 < kstop; k0 += 4) {
-      const int k = k0 + g;
-      float a[NI], b[NI];
+    if (kbeg < kend) load(kbeg);
+    for (int kb = kbeg; kb < kend; ++kb) {
+      ta.store_f32(lds_a);
+      tb.store_f32(lds_b);
+      __syncthreads();
+      if (kb + 1 < kend) load(kb + 1);
 #pragma unroll
-      for (int i = 0; i < NI; ++i) {
-        const int m = wm * WT + i * 16 + c, n = wn * WT + i * 16 + c;
-        a[i] = k < kstop && m < rows ? (AT ? A[(int64_t)k * lda + m] : A[(int64_t)m * lda + k]) : 0.f;
-        b[i] = k < kstop && n < cols ? (BT ? B[(int64_t)n * ldb + k] : B[(int64_t)k * ldb + n]) : 0.f;
+      for (int k = 0; k < XK; k += 4) {
+        float a[NI], b[NI];
+#pragma unroll
+        for (int i = 0; i < NI; ++i) {
+          a[i] = ta.read_f32(lds_a, wm * WT + i * 16 + c, k + g);
+          b[i] = tb.read_f32(lds_b, wn * WT + i * 16 + c, k + g);
+        }
+#pragma unroll
+        for (int i = 0; i < NI; ++i)
+#pragma unroll
+          for (int j = 0; j < NI; ++j) acc[i][j] = mfma_f32_16x16x4(b[j], a[i], acc[i][j]);
       }
-#pragma unroll
-      for (int i = 0; i < NI; ++i)
-#pragma unroll
-        for (int j = 0; j < NI; ++j) acc[i][j] = mfma_f32_16x16x4(b[j], a[i], acc[i][j]);
+      __syncthreads();
     }
   }
 
