@@ -113,3 +113,20 @@ def test_scores_past_the_scaled_range(device, sign):
     got = _layer(x, sign * 2.0 ** -103, causal=True)
     for out, power in {"o": 0, "lse": 0, "dq": -50, "dk": -50, "dv": 0}.items():
         assert T.hybrid_error(np.ldexp(got[out].astype(np.float64), -power), want[out]) <= 1e-4, out
+
+
+def test_scores_of_one_product(device):
+    """One row, q with one nonzero column and a score scale of one in log2 units: L is
+    the rounded product, and O, with P = 1, is V."""
+    rng = np.random.default_rng(8)
+    heads, dim = 600, 64
+    x = _inputs(heads, 1, dim)
+    x["q"][...] = 0.0
+    x["q"][np.arange(heads), 0, rng.integers(0, dim, heads)] = rng.standard_normal(heads, dtype=np.float32)
+    scale = np.float32(np.log(2.0))
+    assert scale * np.float32(1.44269504088896340736) == np.float32(1.0)
+    got = _layer(x, float(scale))
+    exact = np.sum(x["q"][:, 0].astype(np.float64) * x["k"][:, 0], axis=1)
+    ulp = np.exp2(np.floor(np.log2(np.abs(exact))) - 23)
+    assert np.max(np.abs(got["lse"][:, 0] - exact) / ulp) <= 0.52
+    assert np.array_equal(got["o"], x["v"])

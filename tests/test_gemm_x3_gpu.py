@@ -171,3 +171,24 @@ def test_x3_results_past_the_scaled_range(device, layout, m, n, k, power):
     c, got = _run(a, b, layout, 1)
     assert "_x3" in got
     _check(c, a, b, k)
+
+
+@pytest.mark.parametrize("layout", ["nn", "nt", "tn"])
+@pytest.mark.parametrize("m,n,k", [(257, 259, 1025), (1409, 1281, 993)])
+@pytest.mark.parametrize("terms", [1, 2, 4])
+def test_x3_sums_of_few_products(device, layout, m, n, k, terms):
+    """Full-width values, one product to a 32-wide step and `terms` in all: a lone
+    product is within 0.52 of its last place (0.5, and what the seven small partial
+    products, 2^-8 of it, are rounded by), and each further one adds an accumulation
+    of the 16-bit MFMA, whose single steps are up to 0.875 off."""
+    rng = np.random.default_rng(terms)
+    full = lambda *shape: (rng.uniform(1, 2, shape) * np.exp2(rng.integers(-8, 8, shape)) *
+                           rng.choice((-1, 1), shape)).astype(np.float32)
+    a, b = np.zeros((m, k), np.float32), full(k, n)
+    for t in range(terms):
+        a[np.arange(m), (np.arange(m) * 7 + t * (k // terms)) % k] = full(m)
+    c, got = _run(a, b, layout, 1)
+    assert "_x3" in got
+    a64, b64 = a.astype(np.float64), b.astype(np.float64)
+    ulp = np.exp2(np.floor(np.log2(np.abs(a64) @ np.abs(b64))) - 23)
+    assert np.max(np.abs(c - a64 @ b64) / ulp) <= 0.52 + 0.875 * (terms - 1)

@@ -1,7 +1,7 @@
 /*
  * The fp32 attention kernels on the bf16 matrix cores: the generic kernels'
- * work split, ranges and numerics (attn_generic.h) with every product as six bf16
- * MFMAs of three-way split operands (split3.h), which take 3/8 of the fp32 MFMA's
+ * work split, ranges and numerics (attn_generic.h) with every product as eight bf16
+ * MFMAs of three-way split operands (split3.h), which take half the fp32 MFMA's
  * time and round less often.
  *
  * One 256-thread workgroup takes 64 queries (keys in dK/dV), 16 per wave, held in
@@ -11,9 +11,10 @@
  * layout, read by ds_read_b128 and, as the k-major operand, ds_read_b64_tr_b16.
  * Softmax, row sums, P and dS stay fp32; P and dS are split for their products.
  * Measured (us, forward / dQ / dK, dV on the fp32 MFMA and here): 16 heads of 2048
- * rows at 64 columns 194 / 239 / 305 and 144 / 161 / 209, at 128 columns 376 / 475
- * / 666 and 246 / 297 / 464; 2 heads of 96 11.7 / 12.8 / 16.4 and 10.0 / 9.9 /
- * 14.1.  The MFMAs take about half of that time; the rest is the split (5.5 VALU
+ * rows at 64 columns 204 / 239 / 306 and 172 / 190 / 231, at 128 columns 379 / 478
+ * / 669 and 295 / 342 / 569; 2 heads of 96 11.7 / 12.8 / 16.4 and 10.1 / 10.6 /
+ * 14.2 (six products, which lost bits: 160 / 168 / 207, 267 / 296 / 466 and 10.0 /
+ * 9.9 / 14.1).  Beside the MFMAs there is the split (5.5 VALU
  * operations an element and as much again for P and dS) and the LDS round trip
  * between a block's two barriers, which two or three workgroups per CU cover
  * in part.
@@ -155,9 +156,9 @@ TM_DEV void attn_fwd_x3(const TmAttnFwdArgs &p, char *lds) {
   const Lane<DP> at(g, c);
   const float qk_scale = p.sm_scale * TM_LOG2E, s_scale = qk_scale * UNSCALE2;
   float m_i = TM_NEG_INF, l_i = 0.f;
-  f32x4 acc[DT];
+  f32x4 acc[DT], low[DT];
 #pragma unroll
-  for (int dt = 0; dt < DT; ++dt) acc[dt] = (f32x4){0.f, 0.f, 0.f, 0.f};
+  for (int dt = 0; dt < DT; ++dt) acc[dt] = low[dt] = (f32x4){0.f, 0.f, 0.f, 0.f};
 
   const int kend_all = CAUSAL ? min(n, q0 + BM) : n;
   const int nkb = (kend_all + BN - 1) / BN;
@@ -179,17 +180,17 @@ TM_DEV void attn_fwd_x3(const TmAttnFwdArgs &p, char *lds) {
       kr.load(K, k0 + BN, n, D, ss, tid);
       vr.load(V, k0 + BN, n, D, ss, tid);
     }
-    f32x4 s[KT];
+    f32x4 s[KT], sl[KT];
 #pragma unroll
-    for (int kt = 0; kt < KT; ++kt) s[kt] = (f32x4){0.f, 0.f, 0.f, 0.f};
+    for (int kt = 0; kt < KT; ++kt) s[kt] = sl[kt] = (f32x4){0.f, 0.f, 0.f, 0.f};
 #pragma unroll
     for (int ks = 0; ks < KS; ++ks)
 #pragma unroll
       for (int kt = 0; kt < KT; kt += 2) {
-        u32x4 a[3], b[3];
-        row_operand<DP>(kb, at.row[ks], kt * 16, a);
-        row_operand<DP>(kb, at.row[ks], kt * 16 + 16, b);
-        mfma_x3_pair(a, qf[ks], s[kt], b, qf[ks], s[kt + 1]);
+        u32x4 a[2][3];
+        row_operand<DP>(kb, at.row[ks], kt * 16, a[0]);
+        row_operand<DP>(kb, at.row[ks], kt * 16 + 16, a[1]);
+        mfma_x3<2>({&a[0], &a[1]}, {&qf[ks], &qf[ks]}, {&s[kt], &s[kt + 1]}, {&sl[kt], &sl[kt + 1]});
       }
     float mx = TM_NEG_INF;
 #pragma unroll
@@ -197,6 +198,7 @@ TM_DEV void attn_fwd_x3(const TmAttnFwdArgs &p, char *lds) {
 #pragma unroll
       for (int r = 0; r < 4; ++r) {
         const int kj = k0 + kt * 16 + 4 * g + r;
+        s[kt][r] += sl[kt][r];
         note_finite(seen, s[kt][r]);
         float v = s[kt][r] * s_scale;
         if (kj >= n || (CAUSAL && kj > qi)) v = TM_NEG_INF;
@@ -219,17 +221,20 @@ TM_DEV void attn_fwd_x3(const TmAttnFwdArgs &p, char *lds) {
     l_i = l_i * alpha + group4_sum(rs);
     m_i = m_new;
 #pragma unroll
-    for (int dt = 0; dt < DT; ++dt) acc[dt] *= alpha;
+    for (int dt = 0; dt < DT; ++dt) {
+      acc[dt] *= alpha;
+      low[dt] *= alpha;
+    }
 #pragma unroll
     for (int kk = 0; kk < BN / 32; ++kk) {
       u32x4 pf[3];
       result_operand(s[2 * kk], s[2 * kk + 1], X3_SCALE, pf);
 #pragma unroll
       for (int dt = 0; dt < DT; dt += 2) {
-        u32x4 a[3], b[3];
-        k_operand<DP>(vb, at.km[dt], kk * 32, a);
-        k_operand<DP>(vb, at.km[dt + 1], kk * 32, b);
-        mfma_x3_pair(a, pf, acc[dt], b, pf, acc[dt + 1]);
+        u32x4 a[2][3];
+        k_operand<DP>(vb, at.km[dt], kk * 32, a[0]);
+        k_operand<DP>(vb, at.km[dt + 1], kk * 32, a[1]);
+        mfma_x3<2>({&a[0], &a[1]}, {&pf, &pf}, {&acc[dt], &acc[dt + 1]}, {&low[dt], &low[dt + 1]});
       }
     }
   }
@@ -237,7 +242,10 @@ TM_DEV void attn_fwd_x3(const TmAttnFwdArgs &p, char *lds) {
 #pragma unroll
   for (int dt = 0; dt < DT; ++dt)
 #pragma unroll
-    for (int r = 0; r < 4; ++r) beyond |= x3_not_finite(acc[dt][r]);
+    for (int r = 0; r < 4; ++r) {
+      acc[dt][r] += low[dt][r];
+      beyond |= x3_not_finite(acc[dt][r]);
+    }
   if (__syncthreads_or(beyond)) {
     attn_fwd_generic<float, DP, CAUSAL>(p, (float *)lds, (float *)lds + generic_tile(DP));
     return;
@@ -274,6 +282,9 @@ TM_DEV void attn_fwd_x3(const TmAttnFwdArgs &p, char *lds) {
 template <int DP, bool CAUSAL>
 TM_DEV void attn_dq_x3(const TmAttnDqArgs &p, char *lds) {
   constexpr int BM = 64, BN = block_rows(DP), KS = DP / 32, DT = DP / 16;
+  /* the small products' accumulators live through the walk, or (past 64 columns,
+   * where 256 registers do not hold them) through one block */
+  constexpr bool KEEP = DP <= 64;
   const uint32_t kb = lds_addr(lds), vb = kb + planes(DP);
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int g = lane >> 4, c = lane & 15;
@@ -291,9 +302,9 @@ TM_DEV void attn_dq_x3(const TmAttnDqArgs &p, char *lds) {
   const float delta = qi < n ? p.delta[srow] * SCALE2 : 0.f; /* at dP's scale */
   const float qk_scale = p.sm_scale * TM_LOG2E, s_scale = qk_scale * UNSCALE2;
   float seen = 0.f;
-  f32x4 acc[DT];
+  f32x4 acc[DT], low[DT];
 #pragma unroll
-  for (int dt = 0; dt < DT; ++dt) acc[dt] = (f32x4){0.f, 0.f, 0.f, 0.f};
+  for (int dt = 0; dt < DT; ++dt) acc[dt] = low[dt] = (f32x4){0.f, 0.f, 0.f, 0.f};
 
   /* ranges in 32-key blocks, as the generic kernel's: a range's first block may
    * start in the middle of one of BN */
@@ -319,22 +330,26 @@ TM_DEV void attn_dq_x3(const TmAttnDqArgs &p, char *lds) {
 #pragma unroll
     for (int kk = 0; kk < BN / 32; ++kk) {
       if (k0 + kk * 32 >= kend) break; /* the next range's */
-      f32x4 s[2], dp[2];
+      f32x4 s[2], dp[2], sl[2], dpl[2];
       s[0] = s[1] = dp[0] = dp[1] = (f32x4){0.f, 0.f, 0.f, 0.f};
+      sl[0] = sl[1] = dpl[0] = dpl[1] = (f32x4){0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-      for (int ks = 0; ks < KS; ++ks)
+      for (int t = 0; t < 2; ++t)
 #pragma unroll
-        for (int t = 0; t < 2; ++t) {
-          u32x4 a[3], b[3];
-          row_operand<DP>(kb, at.row[ks], kk * 32 + t * 16, a);
-          row_operand<DP>(vb, at.row[ks], kk * 32 + t * 16, b);
-          mfma_x3_pair(a, qf[ks], s[t], b, df[ks], dp[t]);
+        for (int ks = 0; ks < KS; ++ks) {
+          u32x4 a[2][3];
+          row_operand<DP>(kb, at.row[ks], kk * 32 + t * 16, a[0]);
+          row_operand<DP>(vb, at.row[ks], kk * 32 + t * 16, a[1]);
+          mfma_x3<2>({&a[0], &a[1]}, {&qf[ks], &df[ks]}, {&s[t], &dp[t]}, {&sl[t], &dpl[t]});
+          if (DP > 96) __builtin_amdgcn_sched_barrier(0); /* registers: the next reads not yet */
         }
 #pragma unroll
       for (int t = 0; t < 2; ++t)
 #pragma unroll
         for (int r = 0; r < 4; ++r) {
           const int kj = k0 + kk * 32 + t * 16 + 4 * g + r;
+          s[t][r] += sl[t][r];
+          dp[t][r] += dpl[t][r];
           note_finite(seen, s[t][r]);
           float v = s[t][r] * s_scale;
           if (kj >= n || (CAUSAL && kj > qi)) v = TM_NEG_INF;
@@ -344,10 +359,17 @@ TM_DEV void attn_dq_x3(const TmAttnDqArgs &p, char *lds) {
       result_operand(s[0], s[1], 1.f, dsf);
 #pragma unroll
       for (int dt = 0; dt < DT; dt += 2) {
-        u32x4 a[3], b[3];
-        k_operand<DP>(kb, at.km[dt], kk * 32, a);
-        k_operand<DP>(kb, at.km[dt + 1], kk * 32, b);
-        mfma_x3_pair(a, dsf, acc[dt], b, dsf, acc[dt + 1]);
+        u32x4 a[2][3];
+        k_operand<DP>(kb, at.km[dt], kk * 32, a[0]);
+        k_operand<DP>(kb, at.km[dt + 1], kk * 32, a[1]);
+        if constexpr (KEEP) {
+          mfma_x3<2>({&a[0], &a[1]}, {&dsf, &dsf}, {&acc[dt], &acc[dt + 1]}, {&low[dt], &low[dt + 1]});
+        } else {
+          f32x4 l[2] = {};
+          mfma_x3<2>({&a[0], &a[1]}, {&dsf, &dsf}, {&acc[dt], &acc[dt + 1]}, {&l[0], &l[1]});
+          acc[dt] += l[0];
+          acc[dt + 1] += l[1];
+        }
       }
     }
   }
@@ -355,7 +377,10 @@ TM_DEV void attn_dq_x3(const TmAttnDqArgs &p, char *lds) {
 #pragma unroll
   for (int dt = 0; dt < DT; ++dt)
 #pragma unroll
-    for (int r = 0; r < 4; ++r) beyond |= x3_not_finite(acc[dt][r]);
+    for (int r = 0; r < 4; ++r) {
+      acc[dt][r] += low[dt][r];
+      beyond |= x3_not_finite(acc[dt][r]);
+    }
   if (__syncthreads_or(beyond)) {
     attn_dq_generic<float, DP, CAUSAL>(p, (float *)lds, (float *)lds + generic_tile(DP));
     return;
@@ -380,6 +405,8 @@ TM_DEV void attn_dq_x3(const TmAttnDqArgs &p, char *lds) {
 template <int DP, bool CAUSAL>
 TM_DEV void attn_dkdv_x3(const TmAttnDkdvArgs &p, char *lds, float *Ls, float *Ds) {
   constexpr int BN = 64, BM = block_rows(DP), KS = DP / 32, DT = DP / 16;
+  /* one wave per SIMD (past 64 columns) has only its own MFMAs to wait beside */
+  constexpr bool WIDE = DP > 64;
   const uint32_t qb = lds_addr(lds), ob = qb + planes(DP);
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int g = lane >> 4, c = lane & 15;
@@ -395,9 +422,9 @@ TM_DEV void attn_dkdv_x3(const TmAttnDkdvArgs &p, char *lds, float *Ls, float *D
   const Lane<DP> at(g, c);
   const float qk_scale = p.sm_scale * TM_LOG2E, s_scale = qk_scale * UNSCALE2;
   float seen = 0.f;
-  f32x4 dk[DT], dv[DT];
+  f32x4 dk[DT], dv[DT], dkl[DT], dvl[DT];
 #pragma unroll
-  for (int dt = 0; dt < DT; ++dt) dk[dt] = dv[dt] = (f32x4){0.f, 0.f, 0.f, 0.f};
+  for (int dt = 0; dt < DT; ++dt) dk[dt] = dv[dt] = dkl[dt] = dvl[dt] = (f32x4){0.f, 0.f, 0.f, 0.f};
 
   /* ranges in 32-query blocks, as the generic kernel's */
   const int qfirst = CAUSAL ? k0 : 0;
@@ -428,22 +455,31 @@ TM_DEV void attn_dkdv_x3(const TmAttnDkdvArgs &p, char *lds, float *Ls, float *D
 #pragma unroll
     for (int kk = 0; kk < BM / 32; ++kk) {
       if (q0 + kk * 32 >= qstop) break; /* the next range's */
-      f32x4 s[2], dp[2];
+      f32x4 s[2], dp[2], sl[2], dpl[2];
       s[0] = s[1] = dp[0] = dp[1] = (f32x4){0.f, 0.f, 0.f, 0.f};
+      sl[0] = sl[1] = dpl[0] = dpl[1] = (f32x4){0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-      for (int ks = 0; ks < KS; ++ks)
-#pragma unroll
-        for (int t = 0; t < 2; ++t) {
-          u32x4 a[3], b[3];
-          row_operand<DP>(qb, at.row[ks], kk * 32 + t * 16, a);
-          row_operand<DP>(ob, at.row[ks], kk * 32 + t * 16, b);
-          mfma_x3_pair(a, kf[ks], s[t], b, vf[ks], dp[t]);
+      for (int i = 0; i < (WIDE ? KS : 2 * KS); ++i) {
+        const int ks = WIDE ? i : i % KS, t = i / KS;
+        u32x4 a[2][3], b[2][3];
+        row_operand<DP>(qb, at.row[ks], kk * 32 + t * 16, a[0]);
+        row_operand<DP>(ob, at.row[ks], kk * 32 + t * 16, a[1]);
+        if constexpr (WIDE) {
+          row_operand<DP>(qb, at.row[ks], kk * 32 + 16, b[0]);
+          row_operand<DP>(ob, at.row[ks], kk * 32 + 16, b[1]);
+          mfma_x3<4>({&a[0], &a[1], &b[0], &b[1]}, {&kf[ks], &vf[ks], &kf[ks], &vf[ks]},
+                     {&s[0], &dp[0], &s[1], &dp[1]}, {&sl[0], &dpl[0], &sl[1], &dpl[1]});
+        } else {
+          mfma_x3<2>({&a[0], &a[1]}, {&kf[ks], &vf[ks]}, {&s[t], &dp[t]}, {&sl[t], &dpl[t]});
         }
+      }
 #pragma unroll
       for (int t = 0; t < 2; ++t)
 #pragma unroll
         for (int r = 0; r < 4; ++r) {
           const int row = kk * 32 + t * 16 + 4 * g + r, qi = q0 + row;
+          s[t][r] += sl[t][r];
+          dp[t][r] += dpl[t][r];
           note_finite(seen, s[t][r]);
           float v = s[t][r] * s_scale;
           if (qi >= n || (CAUSAL && qi < kj)) v = TM_NEG_INF;
@@ -454,11 +490,18 @@ TM_DEV void attn_dkdv_x3(const TmAttnDkdvArgs &p, char *lds, float *Ls, float *D
       result_operand(s[0], s[1], X3_SCALE, pf);
       result_operand(dp[0], dp[1], 1.f, dsf);
 #pragma unroll
-      for (int dt = 0; dt < DT; ++dt) {
-        u32x4 a[3], b[3];
-        k_operand<DP>(ob, at.km[dt], kk * 32, a);
-        k_operand<DP>(qb, at.km[dt], kk * 32, b);
-        mfma_x3_pair(a, pf, dv[dt], b, dsf, dk[dt]);
+      for (int dt = 0; dt < DT; dt += WIDE ? 2 : 1) {
+        u32x4 a[2][3], b[2][3];
+        k_operand<DP>(ob, at.km[dt], kk * 32, a[0]);
+        k_operand<DP>(qb, at.km[dt], kk * 32, a[1]);
+        if constexpr (WIDE) {
+          k_operand<DP>(ob, at.km[dt + 1], kk * 32, b[0]);
+          k_operand<DP>(qb, at.km[dt + 1], kk * 32, b[1]);
+          mfma_x3<4>({&a[0], &a[1], &b[0], &b[1]}, {&pf, &dsf, &pf, &dsf},
+                     {&dv[dt], &dk[dt], &dv[dt + 1], &dk[dt + 1]}, {&dvl[dt], &dkl[dt], &dvl[dt + 1], &dkl[dt + 1]});
+        } else {
+          mfma_x3<2>({&a[0], &a[1]}, {&pf, &dsf}, {&dv[dt], &dk[dt]}, {&dvl[dt], &dkl[dt]});
+        }
       }
     }
   }
@@ -466,7 +509,11 @@ TM_DEV void attn_dkdv_x3(const TmAttnDkdvArgs &p, char *lds, float *Ls, float *D
 #pragma unroll
   for (int dt = 0; dt < DT; ++dt)
 #pragma unroll
-    for (int r = 0; r < 4; ++r) beyond |= kj < n && (x3_not_finite(dk[dt][r]) || x3_not_finite(dv[dt][r]));
+    for (int r = 0; r < 4; ++r) {
+      dk[dt][r] += dkl[dt][r];
+      dv[dt][r] += dvl[dt][r];
+      beyond |= kj < n && (x3_not_finite(dk[dt][r]) || x3_not_finite(dv[dt][r]));
+    }
   if (__syncthreads_or(beyond)) {
     attn_dkdv_generic<float, DP, CAUSAL>(p, (float *)lds, (float *)lds + generic_tile(DP), Ls, Ds);
     return;

@@ -1,18 +1,19 @@
 /*
  * gfx950 GEMM for fp32 on the bf16 matrix cores: every operand is split into
- * three bf16 parts, x = hi + mid + lo (each the rounding of what is left, 24
- * bits in all), and C = A @ B is the sum of the six products of order 2^-16 and
- * above -- hi hi, hi mid, mid hi, hi lo, mid mid, lo hi -- in one fp32
- * accumulator.  The three dropped products are below 2^-26 of |a b|, less than an
- * fp32 rounding, and a 16x16x32 bf16 MFMA rounds once per 32 products where the
- * 16x16x4 fp32 one rounds once per 4, so the result is no further from the exact
- * one than the fp32 MFMA's; six bf16 MFMAs still take 3/8 of its time.
+ * three bf16 parts (split3.h), and C = A @ B is eight of their nine products, hi hi
+ * in one fp32 accumulator and the seven small ones in another.  A 16x16x32 bf16
+ * MFMA rounds once per 32 products where the 16x16x4 fp32 one rounds per 4, so
+ * dense results are closer to the exact ones than the fp32 MFMA's (relative error
+ * at K = 64, 1025 and 4097: 1.4, 5.7 and 11.4e-7 on that, 0.5, 0.9 and 1.2e-7
+ * here) and a lone product is as close (0.51 of its last place at most, 0.50 on
+ * the fp32 MFMA).  Six products in one accumulator took 15% less time and were up
+ * to 1.41 off there.  Eight bf16 MFMAs take half the fp32 MFMA's time.
  *
  * Measured (us, fp32 MFMA kernels before and now): 2049 x 3079 x 1025 177 and
- * 94, 4096^3 1050 and 725 (190 TFLOP/s), 1500^3 114 and 61, 1000^3 40 and 28,
- * 129 x 202 x 7481 276 and 27.  At 4096^3 the MFMAs take 55% of the time; the rest
- * is what two workgroups per CU leave uncovered of the split (6 VALU operations
- * an element), the LDS writes and transposed reads between its barriers.
+ * 110, 4096^3 1050 and 850, 1500^3 114 and 66, 1000^3 40 and 32, 129 x 202 x 7481
+ * 276 and 27.  Beside the MFMAs there is what two workgroups per CU leave uncovered
+ * of the split (6 VALU operations an element), the LDS writes and transposed reads
+ * between its barriers.
  * Splitting into registers behind the MFMAs instead ran 93 / 738 us, three
  * workgroups per CU (168 registers) 114 / 818.
  *
@@ -46,7 +47,8 @@ template <bool CONTIG, int TILE>
 struct X3Tile {
   static constexpr int TASKS = TILE / 64, CPR = CONTIG ? 4 : TILE / 8, RPT = 256 / CPR;
   static constexpr int PLANE = TILE * XK * 2;
-  uint32_t off[TASKS][2]; /* bytes from the tile's first element */
+  /* bytes from the tile's first element; k-major tasks lie RPT rows apart */
+  uint32_t off[CONTIG ? TASKS : 1][2];
   f32x4 v[TASKS][2];
   int row0, chunk, width;
 
@@ -67,14 +69,16 @@ struct X3Tile {
 #pragma unroll
       for (int t = 0; t < TASKS; ++t)
 #pragma unroll
-        for (int h = 0; h < 2; ++h) v[t][h] = *(const f32x4_any *)(src + off[t][h]);
+        for (int h = 0; h < 2; ++h)
+          v[t][h] = *(const f32x4_any *)(CONTIG ? src + off[t][h] : src + 4 * t * RPT * ld + off[0][h]);
     } else {
 #pragma unroll
       for (int t = 0; t < TASKS; ++t)
 #pragma unroll
         for (int h = 0; h < 2; ++h) {
           const int row = row0 + t * RPT, col = chunk * 8 + h * 4;
-          const f32x4 x = *(const f32x4_any *)(src + x3_last_run<CONTIG>(off[t][h], ld, row, col, k_left));
+          const uint32_t run = CONTIG ? off[t][h] : off[0][h] + 4 * (uint32_t)(t * RPT * ld);
+          const f32x4 x = *(const f32x4_any *)(src + x3_last_run<CONTIG>(run, ld, row, col, k_left));
 #pragma unroll
           for (int e = 0; e < 4; ++e) v[t][h][e] = (CONTIG ? col + e : row) < k_left ? x[e] : 0.f;
         }
@@ -166,11 +170,11 @@ TM_DEV void gemm_x3(const TmGemmArgs &p) {
     ta.load(AT ? A + (int64_t)k0 * lda : A + k0, lda, p.k - k0);
     tb.load(BT ? B + k0 : B + (int64_t)k0 * ldb, ldb, p.k - k0);
   };
-  f32x4 acc[NI][NI];
+  f32x4 acc[NI][NI], low[NI][NI]; /* the hi hi products, the small ones */
 #pragma unroll
   for (int i = 0; i < NI; ++i)
 #pragma unroll
-    for (int j = 0; j < NI; ++j) acc[i][j] = (f32x4){0.f, 0.f, 0.f, 0.f};
+    for (int j = 0; j < NI; ++j) acc[i][j] = low[i][j] = (f32x4){0.f, 0.f, 0.f, 0.f};
 
   if (kbeg < kend) load(kbeg);
   for (int kb = kbeg; kb < kend; ++kb) {
@@ -199,13 +203,14 @@ TM_DEV void gemm_x3(const TmGemmArgs &p) {
                            : *(const u32x4 *)(lds_a + q * PLANE + x3_off(m + c, g));
         af[q] = __builtin_bit_cast(bf16x8, x);
       }
-      /* small products first */
 #pragma unroll
-      for (int order = 2; order >= 0; --order)
+      for (int j = 0; j < NI; ++j) acc[i][j] = mfma_16x16x32(bf[0][j], af[0], acc[i][j]);
 #pragma unroll
-        for (int q = 0; q <= order; ++q)
+      for (int order = 1; order <= 3; ++order)
 #pragma unroll
-          for (int j = 0; j < NI; ++j) acc[i][j] = mfma_16x16x32(bf[q][j], af[order - q], acc[i][j]);
+        for (int q = order < 3 ? 0 : 1; q <= order && q < 3; ++q)
+#pragma unroll
+          for (int j = 0; j < NI; ++j) low[i][j] = mfma_16x16x32(bf[q][j], af[order - q], low[i][j]);
     }
     __syncthreads();
   }
@@ -217,6 +222,7 @@ TM_DEV void gemm_x3(const TmGemmArgs &p) {
     for (int j = 0; j < NI; ++j)
 #pragma unroll
       for (int r = 0; r < 4; ++r) {
+        acc[i][j][r] += low[i][j][r];
         beyond |= x3_not_finite(acc[i][j][r]);
         acc[i][j][r] *= 1.f / (X3_SCALE * X3_SCALE);
       }

@@ -1,7 +1,11 @@
 /* fp32 values as three bf16 parts, x = hi + mid + lo, each the rounding of what
  * is left (24 bits in all): the operands of fp32 products on the bf16 MFMAs
- * (gemm_x3.hip, attn_x3.hip).  A product is the sum of the six of order 2^-16 and
- * above, small ones first; the three dropped are below 2^-26 of it. */
+ * (gemm_x3.hip, attn_x3.hip).  A product is the sum of eight of its nine partial
+ * products, lo lo being below 2^-33 of it: hi hi in one accumulator, the seven
+ * small ones in another, so that a result is rounded at its own magnitude once per
+ * 32 products and a single product within 0.51 of its last place.  (With the six
+ * of order 2^-16 and above in one accumulator a lone product was up to 0.94 of it
+ * off.) */
 #ifndef TM_SPLIT3_H
 #define TM_SPLIT3_H
 
@@ -34,16 +38,22 @@ TM_DEV void x3_split8(float (&x)[8], u32x4 (&part)[3]) {
 constexpr float X3_SCALE = 0x1p16f;
 TM_DEV bool x3_not_finite(float x) { return !(x - x == 0.f); }
 
-/* two products side by side: a product's six MFMAs wait for each other */
-TM_DEV void mfma_x3_pair(const u32x4 (&a0)[3], const u32x4 (&b0)[3], f32x4 &c0, const u32x4 (&a1)[3],
-                         const u32x4 (&b1)[3], f32x4 &c1) {
+/* hi[i], lo[i] += a[i] b[i], N products side by side: one product's seven small
+ * MFMAs wait for each other */
+template <int N>
+TM_DEV void mfma_x3(const u32x4 (*const (&a)[N])[3], const u32x4 (*const (&b)[N])[3], f32x4 *const (&hi)[N],
+                    f32x4 *const (&lo)[N]) {
 #pragma unroll
-  for (int order = 2; order >= 0; --order)
+  for (int i = 0; i < N; ++i)
+    *hi[i] = mfma_16x16x32(__builtin_bit_cast(bf16x8, (*a[i])[0]), __builtin_bit_cast(bf16x8, (*b[i])[0]), *hi[i]);
 #pragma unroll
-    for (int q = order; q >= 0; --q) {
-      c0 = mfma_16x16x32(__builtin_bit_cast(bf16x8, a0[q]), __builtin_bit_cast(bf16x8, b0[order - q]), c0);
-      c1 = mfma_16x16x32(__builtin_bit_cast(bf16x8, a1[q]), __builtin_bit_cast(bf16x8, b1[order - q]), c1);
-    }
+  for (int order = 1; order <= 3; ++order)
+#pragma unroll
+    for (int q = order < 3 ? 0 : 1; q <= order && q < 3; ++q)
+#pragma unroll
+      for (int i = 0; i < N; ++i)
+        *lo[i] = mfma_16x16x32(__builtin_bit_cast(bf16x8, (*a[i])[q]),
+                               __builtin_bit_cast(bf16x8, (*b[i])[order - q]), *lo[i]);
 }
 
 #endif
