@@ -45,13 +45,18 @@ def _check(c, a, b, k):
 
 @pytest.mark.parametrize("layout", ["nn", "nt", "tn"])
 @pytest.mark.parametrize("m,n,k,pad,kernel", [
-    (1, 1, 33, 1, "_t64"),
-    (65, 63, 64, 1, "_t64"),           # whole steps
+    (1, 1, 33, 1, "generic"),          # few tiles of two steps
+    (65, 63, 64, 1, "generic"),
+    (1, 1, 65, 1, "_t64"),
+    (65, 63, 96, 1, "_t64"),           # whole steps
     (129, 257, 65, 3, "_t64"),
     (64, 200, 1000, 2, "_t64"),        # K ranges
-    (1409, 1281, 161, 1, ""),          # 12 x 11 tiles of 128, K ranges
-    (2177, 2050, 95, 1, ""),           # 18 x 17 tiles
-    (2304, 2176, 64, 0, ""),           # whole tiles, more than one per compute unit
+    (1409, 1281, 161, 1, "_t64"),      # 23 x 21 tiles
+    (1409, 1281, 993, 1, ""),          # 12 x 11 tiles of 128, K ranges
+    (2177, 2050, 95, 1, "_t64"),       # 35 x 33 tiles
+    (3585, 3457, 259, 1, ""),          # 29 x 28 tiles of 128
+    (2304, 2176, 64, 0, "_t64"),       # whole tiles, more than one per compute unit
+    (3584, 3584, 256, 0, ""),          # and three of 128 x 128
     (2048, 1024, 1056, 0, ""),         # whole 128 x 128 tiles for half of them, long K
     (128, 320, 512, 0, "_t64"),        # whole 64 x 64 tiles, few
     (1088, 1024, 768, 0, "_t64"),      # and more than one per compute unit
@@ -62,7 +67,7 @@ def test_x3_gemm(device, layout, m, n, k, pad, kernel):
     b = rng.standard_normal((k, n), dtype=np.float32)
     c, got = _run(a, b, layout, pad)
     suffix = "" if layout == "nn" else "_" + layout
-    assert got.split(" + ")[0] == f"tm_gemm_x3{suffix}{kernel}_f32"
+    assert got.split(" + ")[0] == ("tm_gemm_generic_f32" if kernel == "generic" else f"tm_gemm_x3{suffix}{kernel}_f32")
     _check(c, a, b, k)
 
 
@@ -94,7 +99,7 @@ def test_x3_keeps_small_and_large_values(device, layout, scale):
 
 def test_x3_values_that_round_past_bf16(device):
     """3.4e38 rounds to infinity in bf16: the tile is computed in fp32."""
-    m, n, k = 40, 40, 40
+    m, n, k = 40, 40, 70
     a = np.full((m, k), np.float32(3.4e38))
     b = np.zeros((k, n), np.float32)
     b[3] = 0.5
@@ -107,13 +112,13 @@ def test_x3_infinities_and_nan(device):
     """As fp32 arithmetic has them: inf times a number, inf - inf, NaN, and no
     trace in the rows that hold none."""
     rng = np.random.default_rng(2)
-    m, n, k = 70, 66, 50
+    m, n, k = 70, 66, 82
     a = rng.standard_normal((m, k), dtype=np.float32)
     b = np.abs(rng.standard_normal((k, n), dtype=np.float32)) + 0.5
     a[0, 3] = np.inf
     a[1, 4] = -np.inf
     a[2, 5], a[2, 6] = np.inf, -np.inf
-    a[69, 49] = np.nan
+    a[69, 81] = np.nan
     c, got = _run(a, b, "nn", 1)
     assert "_x3" in got
     assert np.all(c[0] == np.inf) and np.all(c[1] == -np.inf)

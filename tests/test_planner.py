@@ -103,3 +103,25 @@ def test_attention_is_planned(limits, element, causal):
         layer.run_backward()
         layer.free()
         _check(limits, (element, causal, dim, heads, seq))
+
+
+@pytest.mark.parametrize("m,n,k,kernel,ranges", [
+    (500, 500, 64, "generic", 1), (500, 500, 65, "x3_t64", 1), (2001, 2001, 64, "x3_t64", 1),
+    (500, 500, 255, "x3_t64", 1), (500, 500, 256, "x3_t64", 2),       # 64 tiles
+    (777, 777, 399, "x3_t64", 1), (777, 777, 400, "x3_t64", 3),       # 169
+    (1001, 1001, 639, "x3_t64", 1), (1001, 1001, 640, "x3_t64", 4),   # 256
+    (1001, 2003, 899, "x3_t64", 2), (1001, 2003, 900, "x3", 4),       # 128 tiles of 128 x 128
+    (2001, 2001, 900, "x3", 2), (2001, 2050, 900, "x3_t64", 1),       # 256, 272
+    (3001, 3001, 4000, "x3_t64", 1),                                  # 576
+    (3585, 3457, 255, "x3_t64", 1), (3585, 3457, 256, "x3", 1),       # 812
+    (16, 32001, 1000, "x3_t64", 2), (150, 20000, 1500, "x3_t64", 1),  # 128 x 128 tiles mostly empty
+])
+def test_fp32_tiles_and_ranges(m, n, k, kernel, ranges):
+    """Each side of the lines between the fp32 GEMM's kernels (choose_gemm_x3,
+    plan_x3_split), at sizes that fill no tile."""
+    planner.launched()
+    _matmul("f32", "nn", m, n, k, 1)
+    launches = planner.launched()
+    assert launches[0][0] == f"tm_gemm_{kernel}_f32"
+    if kernel != "generic":
+        assert launches[0][1][1] == ranges and len(launches) == (2 if ranges > 1 else 1)

@@ -694,10 +694,18 @@ bool gemm_w4_enabled() {
  * few of those, 64 x 64) x 32 tiles runs the fp32 MFMA kernel.  Anything else
  * runs the generic 64 x 64 kernel. */
 /* fp32 on the bf16 matrix cores (gemm_x3.hip): any M, N, 4-byte aligned rows,
- * either operand (not both) stored transposed, K past one 32-wide step (below,
- * the generic kernel: a single step has nothing to overlap).  128 x 128 tiles from half as many as
- * compute units, else 64 x 64 (1500^3 in 144 tiles and 3 ranges 61 us, in 576 of
- * 64 x 64 80). */
+ * either operand (not both) stored transposed, K past one 32-wide step, past two
+ * with at most two 64 x 64 tiles per compute unit (below, the generic kernel: the
+ * steps have nothing to overlap; 500^2, K = 64 5.4 us here and 5.0 there, 1000^2 6.2
+ * and 5.6, 2001^2 11.2 and 12.0).
+ * 128 x 128 or 64 x 64 tiles, us: the large ones where they come in three and more
+ * rounds of one per compute unit, from K = 256 (2500 x 5000 in 800 tiles: K = 256 64
+ * and 64, K = 1000 208 and 230; 6000^2, K = 512 257 and 313), and where half to all
+ * of the compute units have one and a K past 900 splits into ranges (1001 x 2003 in
+ * 128: K = 700 39.5 and 37.4, K = 2000 73.7 and 88; 2001^2 in 256: K = 700 59.5 and
+ * 57.2, K = 2000 131 and 163).  Between, their second round is mostly empty (3001^2
+ * in 576: K = 512 98 and 86, K = 4100 666 and 595).  Not where they cover a quarter
+ * more than the small ones do (16 x 32001, K = 1000: 66.8 and 45.5). */
 bool choose_gemm_x3(Plan &plan, TmGemmArgs &p, const char *family) {
   const bool gemm = strcmp(family, "gemm") == 0;
   if (!fast_paths_enabled() || p.scn != 1 || p.k <= 32) return false;
@@ -708,7 +716,10 @@ bool choose_gemm_x3(Plan &plan, TmGemmArgs &p, const char *family) {
   const bool b_t = !b_n && gemm && p.sbk == 1 && p.sbn >= p.k && p.sbn < limit;
   if (!(a_n && (b_n || b_t)) && !(a_t && b_n)) return false;
   const int64_t cus = std::max(device().compute_units, 1);
-  const bool big = 2 * cdiv(p.m, 128) * cdiv(p.n, 128) >= cus;
+  const int64_t large = cdiv(p.m, 128) * cdiv(p.n, 128), small = cdiv(p.m, 64) * cdiv(p.n, 64);
+  if (p.k <= 64 && small <= 2 * cus) return false;
+  const bool big = 16 * large <= 5 * small &&
+                   (large >= 3 * cus ? p.k >= 256 : large <= cus && 2 * large >= cus && p.k >= 900);
   const int tile = big ? 128 : 64;
   plan.variant = format("tm_%s_x3%s%s_f32", family, b_t ? "_nt" : a_t ? "_tn" : "", big ? "" : "_t64");
   plan.grid[0] = (unsigned)(cdiv(p.m, tile) * cdiv(p.n, tile));
@@ -736,13 +747,12 @@ void choose_gemm(Plan &plan, TmGemmArgs &p, const BuiltinSpec &spec, const char 
     const int64_t tiles = (int64_t)(p.m / tile) * (p.n / tile);
     /* the bf16-split kernel (M, N and K of whole 16-byte runs leave it nothing to
      * read past an operand, whichever tile it takes: x3_runs.h), us against this
-     * one's: more 128 x 128 tiles than
-     * compute units 725 / 1050 (4096^3); up to as many, past K = 1024, 109 / 134
-     * (2048 x 2048 x 1984), 64 / 135 (2048 x 1024 x 2016, B transposed); 64 x 64
-     * tiles for half the compute units, from K = 512 in ranges, 16 / 23 (512 x
-     * 512 x 992), 23 / 111 (64 x 1088 x 5504), or for more than all of them 31 / 38
-     * (1088 x 1024 x 992; at K = 512 23 / 21); between, 28 / 23 (1024 x 1024 x
-     * 992) */
+     * one's: more 128 x 128 tiles than compute units 754 / 1050 (4096^3), 13.4 / 16.8
+     * (2304 x 2176 x 64); up to as many, past K = 1024, 130 / 150 (2048^3), 75 / 136
+     * (2048 x 1024 x 2016, B transposed); 64 x 64 tiles for half the compute units,
+     * from K = 512 in ranges, 17 / 23 (512 x 512 x 992), 24 / 111 (64 x 1088 x 5504),
+     * or for more than all of them 34 / 41 (1088 x 1024 x 992; at K = 512 23 / 21);
+     * between, 32 / 24 (1024 x 1024 x 992) */
     const int64_t cus = std::max(device().compute_units, 1);
     const bool x3 = f32_big ? tiles > cus || p.k > 1024
                             : 2 * tiles <= cus ? p.k >= 512 : tiles > cus && p.k >= 768;
@@ -1007,12 +1017,15 @@ bool plan_x3_split(Plan &plan, TmGemmArgs &p, const Library &lib, const Scratch 
   const int64_t tiles = plan.grid[0], ksteps = cdiv(p.k, 32);
   const bool small = plan.variant.find("_t64") != std::string::npos;
   /* two workgroups of 128 x 128 tiles or four of 64 x 64 per compute unit, at
-   * least four steps to a range (fp32, us without ranges and with: 500^3 18.4
-   * and 11.7, 1000^3 36 and 28, 64 x 1088 x 5504 111 on the generic kernel and
-   * 21, SAE 24 x 3856 x 12352 110 and 55) */
+   * least four steps to a range.  The partials and the reduce dispatch cost more
+   * the more tiles there are, so ranges of 64 x 64 tiles begin at a K that grows
+   * with them; us without and with: 64 tiles (500^2) K = 200 10.5 and 10.7, 256 11.4
+   * and 10.5; 169 (777^2) K = 256 12.2 and 14.0, 400 17.8 and 17.3; 256 (1000^2) K =
+   * 512 21.9 and 24.3, 700 28.9 and 27.7; 484 (1400^2) K = 512 28.9 and 33.2, 700
+   * 39.5 and 39.2 */
   const int64_t target = (small ? 4 : 2) * cus;
   const int64_t splits = std::min<int64_t>({target / tiles, ksteps / 4, 16});
-  if (splits < 2) return false;
+  if (splits < 2 || (small && p.k < (2 * tiles <= cus ? 256 : 4 * tiles <= 3 * cus ? 400 : 640))) return false;
   const int64_t np = (p.n + 3) & ~int64_t(3);
   void *work = plan_workspace(lib, (size_t)splits * (size_t)p.m * (size_t)np * 4, scratch);
   if (!work) return false;
