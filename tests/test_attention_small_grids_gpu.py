@@ -1,5 +1,6 @@
 """The forms that small grids keep: the head_dim 64 dK/dV with one wave per SIMD and
-the fp32 forward on the fp32 MFMAs at 65 to 80 columns, against the fp64 oracle."""
+fp32 attention on the fp32 MFMAs where the split form contracts columns that are not
+there, against the fp64 oracle."""
 
 import math
 
@@ -40,7 +41,7 @@ def test_short_walks_and_larger_grids_take_two_waves(device, heads, seq):
 @pytest.mark.parametrize("causal", [False, True])
 @pytest.mark.parametrize("heads,seq,dim,pad,kept", [
     (2, 1, 80, 0, True), (3, 65, 65, 1, True), (6, 113, 80, 3, True), (2, 512, 72, 0, True),
-    (2, 513, 80, 0, False), (2, 100, 81, 0, False), (65, 128, 80, 0, False),
+    (2, 513, 80, 0, True), (2, 100, 81, 0, True), (65, 128, 80, 0, False), (5, 513, 80, 0, False),
 ])
 def test_fp32_forward_65_to_80(device, heads, seq, dim, pad, causal, kept):
     out, variants, dense, _ = _attention(heads, seq, dim, "f32", causal, stride_seq=dim + pad)
@@ -48,3 +49,23 @@ def test_fp32_forward_65_to_80(device, heads, seq, dim, pad, causal, kept):
     want = R.attention_backward(*dense, 1 / math.sqrt(dim), causal)
     assert T.hybrid_error(out["o"], want["o"]) <= 2e-5
     assert T.hybrid_error(out["lse"], want["lse"]) <= 2e-5
+
+
+@pytest.mark.parametrize("causal", [False, True])
+@pytest.mark.parametrize("heads,seq,dim,pad,kept", [
+    # forward, dQ, dK/dV on the fp32 MFMAs
+    (2, 97, 5, 2, "111"), (1, 1000, 20, 0, "111"), (6, 113, 40, 0, "111"),   # small, at most 40 columns
+    (2, 97, 41, 1, "100"), (3, 65, 88, 0, "101"), (2, 96, 103, 1, "101"),    # the forward, dK/dV past 64
+    (1, 129, 111, 1, "100"), (1, 129, 112, 0, "000"), (2, 96, 64, 0, "000"),
+    (24, 300, 33, 0, "000"), (50, 150, 5, 2, "000"),                         # larger
+    (24, 300, 72, 4, "101"), (24, 300, 81, 1, "001"), (24, 300, 104, 0, "000"), (24, 300, 96, 0, "000"),
+])
+def test_fp32_kernels_by_head_dimension(device, heads, seq, dim, pad, causal, kept):
+    out, variants, dense, _ = _attention(heads, seq, dim, "f32", causal, stride_seq=dim + pad)
+    names = (variants[0], variants[2], variants[3])
+    assert "".join(str(int("_mfma32" in v)) for v in names) == kept, variants
+    want = R.attention_backward(*dense, 1 / math.sqrt(dim), causal)
+    assert T.hybrid_error(out["o"], want["o"]) <= 2e-5
+    assert T.hybrid_error(out["lse"], want["lse"]) <= 2e-5
+    for name in ("dq", "dk", "dv"):
+        assert T.hybrid_error(out[name], want[name]) <= 1e-4, name

@@ -189,33 +189,28 @@ TM_PRE(float, tm_attn_pre_generic_f32)
 TM_PRE(f16_t, tm_attn_pre_generic_f16)
 TM_PRE(bf16_t, tm_attn_pre_generic_bf16)
 
-/* the fp32 forward on the fp32 MFMAs, beside attn_x3.hip's (65 to 80 columns, short
- * sequences of few heads) */
-#define TM_FWD_F32(DP, CAUSAL, CN)                                                            \
-  extern "C" __global__ __launch_bounds__(256) void tm_attn_fwd_generic_f32_d##DP##CN##_mfma32( \
-      TmAttnFwdArgs p) {                                                                      \
-    __shared__ __align__(16) float k[generic_tile(DP)], v[generic_tile(DP)];                  \
-    attn_fwd_generic<float, DP, CAUSAL>(p, k, v);                                             \
-  }
-TM_FWD_F32(96, false, )
-TM_FWD_F32(96, true, _causal)
-
-#define TM_ATTN_ONE(T, TN, DP, CAUSAL, CN)                                                    \
+#define TM_ATTN_FWD(T, TN, DP, CAUSAL, CN)                                                    \
   extern "C" __global__ __launch_bounds__(256) void tm_attn_fwd_generic_##TN##_d##DP##CN(     \
       TmAttnFwdArgs p) {                                                                      \
     __shared__ __align__(16) float k[generic_tile(DP)], v[generic_tile(DP)];                  \
     attn_fwd_generic<T, DP, CAUSAL>(p, k, v);                                                 \
-  }                                                                                           \
+  }
+#define TM_ATTN_DQ(T, TN, DP, CAUSAL, CN)                                                     \
   extern "C" __global__ __launch_bounds__(256) void tm_attn_dq_generic_##TN##_d##DP##CN(      \
       TmAttnDqArgs p) {                                                                       \
     __shared__ float k[32 * (DP + 1)], v[32 * (DP + 1)];                                      \
     attn_dq_generic<T, DP, CAUSAL>(p, k, v);                                                  \
-  }                                                                                           \
+  }
+#define TM_ATTN_DKDV(T, TN, DP, CAUSAL, CN)                                                   \
   extern "C" __global__ __launch_bounds__(256) void tm_attn_dkdv_generic_##TN##_d##DP##CN(    \
       TmAttnDkdvArgs p) {                                                                     \
     __shared__ float q[32 * (DP + 1)], d[32 * (DP + 1)], l[32], dl[32];                       \
     attn_dkdv_generic<T, DP, CAUSAL>(p, q, d, l, dl);                                         \
   }
+#define TM_ATTN_ONE(T, TN, DP, CAUSAL, CN) \
+  TM_ATTN_FWD(T, TN, DP, CAUSAL, CN)       \
+  TM_ATTN_DQ(T, TN, DP, CAUSAL, CN)        \
+  TM_ATTN_DKDV(T, TN, DP, CAUSAL, CN)
 #define TM_ATTN_DT(T, TN, DP)        \
   TM_ATTN_ONE(T, TN, DP, false, )    \
   TM_ATTN_ONE(T, TN, DP, true, _causal)
@@ -226,3 +221,18 @@ TM_FWD_F32(96, true, _causal)
   TM_ATTN_DT(T, TN, 128)
 TM_ATTN_ALL_DP(f16_t, f16)
 TM_ATTN_ALL_DP(bf16_t, bf16)
+/* fp32 on the fp32 MFMAs, beside attn_x3.hip's: the head dimensions and problem
+ * sizes that the planner keeps here (attn_fp32_mfma in runtime.cpp) */
+#define TM_ATTN_MFMA32(NAME, DP)                   \
+  TM_ATTN_##NAME(float, f32, DP, false, _mfma32)   \
+  TM_ATTN_##NAME(float, f32, DP, true, _causal_mfma32)
+TM_ATTN_MFMA32(FWD, 32)
+TM_ATTN_MFMA32(FWD, 64)
+TM_ATTN_MFMA32(FWD, 96)
+TM_ATTN_MFMA32(FWD, 128)
+TM_ATTN_MFMA32(DQ, 32)
+TM_ATTN_MFMA32(DQ, 64)
+TM_ATTN_MFMA32(DKDV, 32)
+TM_ATTN_MFMA32(DKDV, 64)
+TM_ATTN_MFMA32(DKDV, 96)
+TM_ATTN_MFMA32(DKDV, 128)

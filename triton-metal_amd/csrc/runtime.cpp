@@ -1068,15 +1068,32 @@ int64_t fast_ranges(int64_t wgs, int64_t n_ctx, int head_dim) {
   return std::max<int64_t>(1, std::min<int64_t>({2 * cus / wgs, n_ctx / 256, 16}));
 }
 
-/* Where the fp32 forward keeps the fp32 MFMAs: at 65 to 80 columns the split form
- * contracts 96, which costs more than the faster MFMAs save while a grid leaves
- * half the compute units idle (`wgs` workgroups of 64 queries) and walks at most
- * 512 keys.  us, fp32 MFMA and split, 80 columns: 6 heads of 113 rows 14.7 and
- * 15.7, 16 of 256 19.1 and 20.1, 4 of 512 17.9 and 19.1; 40 of 300 49.7 and 47.1;
- * 4 of 600 28.5 and 26.8; 96 columns, 16 of 256 20.5 and 19.0. */
-bool fwd_fp32_mfma(const BuiltinSpec &spec, int64_t wgs, int64_t n_ctx) {
-  return spec.element == Element::F32 && spec.head_dim > 64 && spec.head_dim <= 80 &&
-         n_ctx <= 512 && 2 * wgs <= device().compute_units;
+/* Where fp32 attention keeps the fp32 MFMAs (generic.hip, `wgs` workgroups of 64
+ * rows): the split form contracts whole 32 columns, the fp32 one only those there
+ * are, and its walk is shorter at first.  us, fp32 MFMA and split:
+ *  - small problems at head dimensions that are no multiple of 32: 2 heads of 96
+ *    rows at 20 columns 6.4 / 6.2 / 7.9 and 7.4 / 7.5 / 9.5 (forward, dQ, dK/dV), 16
+ *    of 256 11.2 / 10.4 / 14.1 and 12.0 / 11.1 / 14.8; 1 of 1000 at 40 columns 13.7 /
+ *    13.9 / 18.5 and 14.7 / 14.2 / 19.2, at 56 columns 15.4 / 15.0 / 19.8 and 16.0 /
+ *    14.6 / 19.4; 2 heads of 1000 at 40 columns 22.0 / 25.1 / 31.5 and 21.1 / 21.6 /
+ *    28.4; the forward of 2 heads of 96 at 88 columns 13.7 and 15.2, at 112 16.0 and 15.7;
+ *  - the forward of 65 to 80 columns up to half the compute units and 512 keys: 16
+ *    of 256 19.1 and 20.1, 4 of 512 17.9 and 19.1; 40 of 300 49.7 and 47.1;
+ *  - dK/dV of 65 to 103 columns but 96, one wave per SIMD in the split form: 32 heads
+ *    of 1000 at 80 columns 271 and 282, at 100 342 and 366, at 104 343 and 316. */
+enum class AttnOp { Fwd, Dq, Dkdv };
+bool attn_fp32_mfma(const BuiltinSpec &spec, AttnOp op, int64_t wgs, int64_t n_ctx) {
+  const int d = spec.head_dim;
+  if (spec.element != Element::F32 || d % 32 == 0) return false;
+  const bool short_grid = 2 * wgs <= device().compute_units, small = short_grid && wgs * n_ctx <= 20000;
+  switch (op) {
+    case AttnOp::Fwd:
+      return (small && d < 112) ||
+             (short_grid && d > 64 && d <= 80 && n_ctx <= 512);
+    case AttnOp::Dq: return small && d <= 40;
+    case AttnOp::Dkdv: return (small && d <= 40) || (d > 64 && d < 104);
+  }
+  return false;
 }
 
 /* Where the head_dim 64 dK/dV runs one wave per SIMD (attn_dkdv_1w): a grid of one
@@ -1256,7 +1273,8 @@ Plan plan_builtin(Kernel &k, const Library &lib, const std::vector<Arg> &args, i
         plan.variant = attn_symbol("fwd", spec);
         plan.grid[0] = (unsigned)cdiv(p.n_ctx, 64);
         plan.grid[1] = (unsigned)heads;
-        if (fwd_fp32_mfma(spec, (int64_t)plan.grid[0] * heads, p.n_ctx)) plan.variant += "_mfma32";
+        if (attn_fp32_mfma(spec, AttnOp::Fwd, (int64_t)plan.grid[0] * heads, p.n_ctx))
+          plan.variant += "_mfma32";
         plan.block = 256;
         /* Too few 64-query workgroups to fill the chip twice, each walking
          * many key blocks: split every workgroup's key blocks into `splits`
@@ -1386,6 +1404,7 @@ Plan plan_builtin(Kernel &k, const Library &lib, const std::vector<Arg> &args, i
         p.head_dim = spec.head_dim;
         p.heads = (int32_t)heads;
         plan.variant = fast ? fast_name : attn_symbol("dq", spec);
+        if (attn_fp32_mfma(spec, AttnOp::Dq, (int64_t)plan.grid[0] * heads, n_ctx)) plan.variant += "_mfma32";
         const int64_t splits = fast ? fast_ranges(plan.grid[0], n_ctx, spec.head_dim)
                                     : split_ranges((int64_t)plan.grid[0] * heads, n_ctx);
         void *work = splits > 1 ? plan_workspace(lib, (size_t)splits * (size_t)heads * (size_t)n_ctx *
@@ -1415,6 +1434,7 @@ Plan plan_builtin(Kernel &k, const Library &lib, const std::vector<Arg> &args, i
         p.head_dim = spec.head_dim;
         p.heads = (int32_t)heads;
         plan.variant = fast ? fast_name : attn_symbol("dkdv", spec);
+        if (attn_fp32_mfma(spec, AttnOp::Dkdv, (int64_t)plan.grid[0] * heads, n_ctx)) plan.variant += "_mfma32";
         const int64_t splits = fast ? fast_ranges(plan.grid[0], n_ctx, spec.head_dim)
                                     : split_ranges((int64_t)plan.grid[0] * heads, n_ctx);
         void *work = splits > 1 ? plan_workspace(lib, (size_t)splits * 2 * (size_t)heads *
