@@ -99,3 +99,24 @@ def test_offsets_move_when_scores_grow(device):
     want_o, _, want_l = R.attention_forward(q, k, v, 1 / math.sqrt(dim), False)
     assert T.max_abs_error(o, want_o) <= 4e-3
     assert T.hybrid_error(lse, want_l) <= 2e-5
+
+
+@pytest.mark.parametrize("dim", [32, 80, 120])
+def test_small_probabilities_keep_their_bits(device, dim):
+    """f16 holds P unscaled: 89 x 2^-24, a value of f16, for every key but the first,
+    which holds the row maximum and a V of 0."""
+    heads, seq = 4, 512
+    q, k = (np.zeros((heads, seq, dim), np.float32) for _ in range(2))
+    q[:, :, 0] = 1.0
+    k[:, 1:, 0] = -1.0
+    v = np.ones((heads, seq, dim), np.float32)
+    v[:, 0] = 0.0
+    layer = ops.AttentionLayer(heads, seq, dim, "f16", scale=math.log(2.0 ** 24 / 89))
+    try:
+        o, _ = layer.forward(q, k, v)
+        assert "_generic_f16_p" in _core.kernel_variant(layer.lib.kernels["attn_fwd"])
+    finally:
+        layer.free()
+    p = 89 * 2.0 ** -24
+    want = (seq - 1) * p / (1 + (seq - 1) * p)
+    assert np.max(np.abs(o - want)) <= 2e-3 * want  # the rounding of O is 2^-11, a bias of 2^-2 11e-3

@@ -332,10 +332,15 @@ struct TileCopy {
  * block take its exact row maxima, move the offsets and redo its P.  bf16 has
  * fp32's exponent range, so B = 32 lets the offset lag the maximum by 33 with
  * no value near overflow; f16's range allows B = 2.  O = acc / l and
- * L = mb + log2(l) are unchanged by any choice of offsets. */
-template <typename T> struct PBias;
-template <> struct PBias<bf16_t> { static constexpr float B = 32.f; };
-template <> struct PBias<f16_t> { static constexpr float B = 2.f; };
+ * L = mb + log2(l) are unchanged by any choice of offsets.
+ * PAD f16: B = 0.  The generic kernels, whose numerics these carry, hold P
+ * unscaled, normal from 2^-14; a bias of 2 would leave it subnormal from 2^-12.
+ * There a packed maximum takes the place of the OR, for a limit of 2^9 (at 2, an
+ * offset would move for every growth by a factor of two: the forward of 4 heads of
+ * 2048 rows at 80 columns 77 us, so 33). */
+template <typename T, bool PAD = false> struct PBias;
+template <bool PAD> struct PBias<bf16_t, PAD> { static constexpr float B = 32.f, UNBIAS = 4294967296.f; /* 2^B */ };
+template <bool PAD> struct PBias<f16_t, PAD> { static constexpr float B = PAD ? 0.f : 2.f, UNBIAS = PAD ? 1.f : 4.f; };
 
 /* PAD: the row sums are fp32 sums of the unrounded P, kept per lane beside the
  * exponentials (the generic kernels' l, so L stays as exact as theirs), instead
@@ -352,7 +357,8 @@ TM_DEV void attn_fwd_fast(const TmAttnFwdArgs &p) {
   constexpr int NM2 = PT * KK * QT;     /* P V MFMAs per block, row sums included */
   constexpr int VS = QT * BN / 2;       /* softmax slots per iteration (4 per element pair) */
   constexpr int LA = 2;                 /* operands read ahead */
-  constexpr float BIAS = PBias<T>::B;
+  constexpr float BIAS = PBias<T, PAD>::B;
+  constexpr bool UNSCALED = BIAS == 0.f;
   __shared__ __align__(1024) char lds[4 * TILE];
   const uint32_t kb0 = lds_addr(lds), kb1 = kb0 + TILE, vb0 = kb0 + 2 * TILE, vb1 = kb0 + 3 * TILE;
 
@@ -535,7 +541,7 @@ TM_DEV void attn_fwd_fast(const TmAttnFwdArgs &p) {
     };
     /* softmax slot v: element pair u = v / 4 (elements 2w, 2w+1 of [qt][kk])
      * as fma, exp, pack and OR on four consecutive slots */
-    uint32_t big = 0;       /* OR of the packed P words */
+    uint32_t big = 0;       /* OR (UNSCALED: maximum) of the packed P words */
     float px[2], pe[2];
     float lprev[QT]; /* PAD: the sums before this block, should it be redone */
 #pragma unroll
@@ -563,6 +569,10 @@ TM_DEV void attn_fwd_fast(const TmAttnFwdArgs &p) {
           lsum[qt] += pe[0] + pe[1];
           pin(lsum[qt]);
         }
+      } else if constexpr (UNSCALED) {
+        typedef unsigned short us2 __attribute__((ext_vector_type(2)));
+        big = __builtin_bit_cast(uint32_t, __builtin_elementwise_max(__builtin_bit_cast(us2, big), __builtin_bit_cast(us2, wd)));
+        pin(big);
       } else if constexpr (u % 2 == 0) {
         wprev = wd; /* ORed with the next pair's word: one v_or3 per two words */
       } else {
@@ -601,11 +611,12 @@ TM_DEV void attn_fwd_fast(const TmAttnFwdArgs &p) {
       TM_FENCE();
     });
     if constexpr (SM) {
-      /* some P reached 2: recompute this block's scores with K fragments read
+      /* some P reached 2 (UNSCALED: 2^9, the upper two exponent bits): recompute this block's scores with K fragments read
        * straight from HBM (its tile is being overwritten and its scores are no
        * longer in registers), take the exact row maxima, move the offsets,
        * redo P, and scale O and the row sums, which hold the P V of every
        * block computed under the old offsets (all issued above) */
+      if (UNSCALED) big &= big << 1;
       if (__builtin_amdgcn_ballot_w64((big & 0x40004000u) != 0) != 0) {
         f32x4 sr[KT][QT];
         scores(sr, [&](int kt, int ks) {
@@ -694,11 +705,9 @@ TM_DEV void attn_fwd_fast(const TmAttnFwdArgs &p) {
       }
       /* PAD: the bias taken out of both terms first (exactly), so L is not
        * rounded at the bias's magnitude */
-      constexpr float UNBIAS = PBias<T>::B == 32.f ? 4294967296.f : 4.f;
-      static_assert(PBias<T>::B == 32.f || PBias<T>::B == 2.f, "UNBIAS = 2^B");
       if (p.lse && g == 0)
         p.lse[(int64_t)bh * p.stride_lse + qi] =
-            PAD ? (mb[qt] - BIAS) + log2f(l * UNBIAS) : mb[qt] + log2f(l);
+            PAD ? (mb[qt] - BIAS) + log2f(l * PBias<T, PAD>::UNBIAS) : mb[qt] + log2f(l);
     }
   }
 }
