@@ -125,3 +125,22 @@ def test_fp32_tiles_and_ranges(m, n, k, kernel, ranges):
     assert launches[0][0] == f"tm_gemm_{kernel}_f32"
     if kernel != "generic":
         assert launches[0][1][1] == ranges and len(launches) == (2 if ranges > 1 else 1)
+
+
+@pytest.mark.parametrize("layout", ["nn", "nt", "tn"])
+def test_wave_groups(limits, layout):
+    """Waves a workgroup of the 16-bit 64 x 64 and 128 x 128 kernels has (two and four
+    to a K group) on each side of the lines between one, two and four groups."""
+    for m, n, k, groups in ((520, 520, 192, 1), (520, 520, 193, 2), (520, 520, 256, 2), (520, 520, 257, 4),
+                            (1400, 1400, 255, 1), (1400, 1400, 256, 2),
+                            (512, 512, 128, 4 if layout == "nn" else 1), (512, 512, 192, 4)):
+        planner.launched()
+        _matmul("bf16", layout, m, n, k, 8 if k % 8 == 0 else (-k) % 8 + 8)
+        name, _, threads, _ = planner.launched()[0]
+        assert threads == 128 * groups, (m, n, k, name, threads)
+    for m, n, k, groups in ((2048, 2048, 128, 2 if layout == "nn" else 1), (2048, 2048, 192, 2),
+                            (2304, 2176, 512, 2 if layout == "nn" else 1)):
+        planner.launched()
+        _matmul("bf16", layout, m, n, k)
+        name, _, threads, _ = planner.launched()[0]
+        assert "_t128" in name and threads == 256 * groups, (m, n, k, name, threads)

@@ -817,23 +817,30 @@ void choose_gemm(Plan &plan, TmGemmArgs &p, const BuiltinSpec &spec, const char 
     const bool whole =
         aligned && p.m % tile == 0 && p.n % tile == 0 && p.k % 64 == 0 && p.scm % 4 == 0;
     const int64_t tiles = cdiv(p.m, tile) * cdiv(p.n, tile);
-    /* fewer 128 x 128 workgroups than two per CU (one wave per SIMD), or 64 x
-     * 64 ones (two waves each): the K loop split over wave groups inside the
-     * workgroup -- whole 128 x 128 tiles over 2 (512 threads); 64 x 64 tiles
-     * over 4 (512 threads, one workgroup per CU) up to one tile per CU, else
+    /* few 128 x 128 workgroups (one wave per SIMD), or at most two 64 x 64 ones per
+     * CU (two waves each): the K loop split over wave groups inside the workgroup --
+     * whole 128 x 128 tiles over 2 (512 threads), with an operand transposed up to one
+     * per CU, as a further one's LDS waits for a second round (2304 x 2176 x 512, B
+     * transposed 18.1 us, 16.2 on one group), row-major up to two (18.4 and 16.2); 64
+     * x 64 tiles over 4 (512 threads, one workgroup per CU) up to one tile per CU, else
      * over 2 (256 threads, two per CU) up to two.  1024^3 f16 with B or A
      * transposed: 16.9 us on one group and 4 K ranges, 6.4 on four groups;
-     * 1000^3 18.4 and 9.4; 2048^3 with B transposed 29.1 and 22.5.  Ragged and
+     * 1000^3 18.4 and 9.4; 2048^3 with B transposed 29.1 and 22.5; 1024^2 x 128 B
+     * transposed 3.9 on one and 4.4 on four.  Ragged and
      * unaligned matmuls of few tiles, or of one tile row (bound by reading B:
      * 16 x 8192 x 8192 35.0 us, 35.7 on four groups), and more than twelve
      * k-steps keep one group and split K across workgroups (plan_gemm_split),
-     * which the SAE encoder does not; over 2 groups they need four k-steps (1400 x 1400 x 136: 6.4 on
-     * one, 6.8 on two). */
+     * which the SAE encoder does not.  Up to three k-steps they keep one group, four
+     * they split over two (520 x 520, us on 1, 2 and 4: K = 160 5.7, 5.9, 6.5, with B
+     * transposed 5.7, 5.7, 6.3; K = 200 6.2, 5.7, 6.4 and 6.2, 5.7, 6.3; K = 330 6.7,
+     * 6.7, 6.7 and 6.6, 5.9, 5.8); over 2 groups of more tiles than CUs they need four
+     * (1400 x 1400 x 136: 6.4 on one, 6.8 on two). */
+    const int64_t ksteps = cdiv(p.k, 64);
     const bool ksplit = TM_GEMM_KSPLIT && !big &&
-                        (small ? tiles <= 2 * cus : tiles < 2 * cus) &&
-                        p.k >= (whole || tiles <= cus ? 128 : 256) &&
+                        (small ? tiles <= 2 * cus : nn ? tiles < 2 * cus : tiles <= cus) &&
+                        p.k >= (whole ? (nn ? 128 : 192) : tiles <= cus ? 193 : 256) &&
                         (whole || (small && (!gemm || (4 * tiles > cus && p.m > 64) || p.k <= 768)));
-    const int kg = !ksplit ? 1 : small && tiles > cus ? 2 : small ? 4 : 2;
+    const int kg = !ksplit ? 1 : !small || tiles > cus || (!whole && ksteps == 4) ? 2 : 4;
     /* the kernels that take their K groups from the launch, and their further
      * groups' LDS (the aligned ones hold one group's tiles themselves); of many
      * tiles, one group each, the kernel of its own */
