@@ -127,6 +127,26 @@ def test_fp32_tiles_and_ranges(m, n, k, kernel, ranges):
         assert launches[0][1][1] == ranges and len(launches) == (2 if ranges > 1 else 1)
 
 
+def test_padded_forward_of_one_head(limits):
+    """One long head of few columns: the generic forward in ranges, the padded
+    backward; otherwise padded throughout from four workgroups on."""
+    ops, _ = planner.package()
+    for heads, seq, dim, forward, backward in (
+            (1, 800, 32, "p32", "p32"), (1, 801, 32, "d32", "p32"), (1, 3000, 32, "d32", "p32"),
+            (1, 3001, 32, "p32", "p32"), (2, 1000, 32, "p32", "p32"), (1, 1000, 56, "d64", "p64"),
+            (1, 2049, 56, "p64", "p64"), (1, 1000, 72, "p80", "p80"), (1, 384, 80, "d96", "d96"),
+            (1, 385, 80, "p80", "p80"), (4, 1, 80, "p80", "p80")):
+        layer = ops.AttentionLayer(heads, seq, dim, "bf16")
+        planner.launched()
+        layer.run_forward()
+        fwd = planner.launched()[0][0]
+        layer.run_backward()
+        bwd = [x[0] for x in planner.launched() if "_dq_" in x[0] or "_dkdv_" in x[0]]
+        layer.free()
+        assert fwd == f"tm_attn_fwd_generic_bf16_{forward}", (heads, seq, dim, fwd)
+        assert len(bwd) == 2 and all(f"_generic_bf16_{backward}" in b for b in bwd), (heads, seq, dim, bwd)
+
+
 @pytest.mark.parametrize("layout", ["nn", "nt", "tn"])
 def test_wave_groups(limits, layout):
     """Waves a workgroup of the 16-bit 64 x 64 and 128 x 128 kernels has (two and four

@@ -53,14 +53,6 @@
 #define TM_FWD_FAST_THREADS 256
 #endif
 
-/* Fewest 128-row workgroups for which the padded 16-bit attention kernels run
- * (forward + backward, bf16 causal: 4 heads of 128 rows at head_dim 80 26 us
- * against the generic kernels' 74; one head of 300 rows keeps the generic
- * kernels' ranges) */
-#ifndef TM_ATTN_PAD_MIN
-#define TM_ATTN_PAD_MIN 4
-#endif
-
 namespace {
 
 /* ---- errors ----------------------------------------------------------------
@@ -610,19 +602,33 @@ bool attn_fast_ok(const BuiltinSpec &spec, int32_t stride_head, int32_t stride_s
 }
 
 /* Other head dimensions that are multiples of 8 run the same kernels padded
- * (attn_pad.hip), contracted at this many columns; 0: the generic kernels.
- * Their workgroups take 128 rows and do not split into ranges, so the smallest
- * grids stay with the generic kernels, whose ranges fill the chip. */
+ * (attn_pad.hip), contracted at this many columns; 0: the generic kernels, which
+ * keep grids of fewer than four 128-row workgroups and split them into ranges (us,
+ * forward, dQ, dK/dV, padded and generic: 4 heads of 64 rows at 80 columns 4.4 / 4.1
+ * / 5.2 and 15.5 / 17.8 / 23.0; below the line padded is the faster one too, 1 head of
+ * 300 rows 8.5 / 8.9 / 12.4 and 20.1 / 21.4 / 27.9). */
 int attn_pad_width(const BuiltinSpec &spec, int64_t heads, int32_t stride_head, int32_t stride_seq,
                    int32_t n_ctx, float sm_scale) {
   const int d = spec.head_dim;
-  if (d == 64 || d == 128 || d % 8 || cdiv(n_ctx, 128) * heads < TM_ATTN_PAD_MIN ||
+  if (d == 64 || d == 128 || d % 8 || cdiv(n_ctx, 128) * heads < 4 ||
       !attn_half_ok(spec, stride_head, stride_seq, n_ctx, sm_scale))
     return 0;
-  /* one long head at 32 columns: the generic kernels' ranges win (1 x 2000 at
-   * head_dim 32: 72 against 91 us; 2 x 1000: 58 against 54) */
-  if (d <= 32 && heads == 1 && n_ctx > 512) return 0;
   return d <= 32 ? 32 : d <= 64 ? 64 : d <= 80 ? 80 : d <= 96 ? 96 : 128;
+}
+
+/* The forward, whose padded form does not split into ranges, keeps the generic
+ * kernels' for one long head of few columns.  us, padded and generic ranges: 32
+ * columns, 800 rows 11.7 and 12.8 (causal 12.5 and 12.2), 1000 13.5 and 11.8, 2000
+ * 24.1 and 20.0, 3000 33.9 and 35.0 (causal 33.9 and 27.4), 4000 44.4 and 49.5; 40
+ * columns, 1000 15.2 and 14.2, 2000 26.9 and 25.5, 3000 37.7 and 51.5; 80 columns,
+ * 1000 18.0 and 23.5; two heads of 1000 at 32 columns 13.8 and 16.2.  (dQ and dK/dV
+ * have ranges of their own: one head of 1000 at 32 columns 10.2 and 11.7, 13.3 and
+ * 15.7, of 2000 10.8 and 21.8, 14.7 and 28.3.) */
+int attn_fwd_pad_width(const BuiltinSpec &spec, int64_t heads, int32_t stride_head, int32_t stride_seq,
+                       int32_t n_ctx, float sm_scale) {
+  if (heads == 1 && n_ctx > 800 && (spec.head_dim <= 32 ? n_ctx <= 3000 : spec.head_dim <= 56 && n_ctx <= 2048))
+    return 0;
+  return attn_pad_width(spec, heads, stride_head, stride_seq, n_ctx, sm_scale);
 }
 
 int padded_head_dim(int d) { return d <= 32 ? 32 : d <= 64 ? 64 : d <= 96 ? 96 : 128; }
@@ -1271,8 +1277,8 @@ Plan plan_builtin(Kernel &k, const Library &lib, const std::vector<Arg> &args, i
                               spec.causal ? "_causal" : "");
         plan.grid[0] = (unsigned)(cdiv(p.n_ctx, TM_FWD_FAST_ROWS) * heads);
         plan.block = TM_FWD_FAST_THREADS;
-      } else if (const int width = attn_pad_width(spec, heads, p.stride_head, p.stride_seq,
-                                                  p.n_ctx, p.sm_scale)) {
+      } else if (const int width = attn_fwd_pad_width(spec, heads, p.stride_head, p.stride_seq,
+                                                      p.n_ctx, p.sm_scale)) {
         plan.variant = attn_pad_symbol("fwd", spec, width);
         plan.grid[0] = (unsigned)(cdiv(p.n_ctx, TM_FWD_FAST_ROWS) * heads);
         plan.block = TM_FWD_FAST_THREADS;
