@@ -113,7 +113,8 @@ def test_attention_is_planned(limits, element, causal):
     (1001, 2003, 899, "x3_t64", 2), (1001, 2003, 900, "x3", 4),       # 128 tiles of 128 x 128
     (2001, 2001, 900, "x3", 2), (2001, 2050, 900, "x3_t64", 1),       # 256, 272
     (3001, 3001, 4000, "x3_t64", 1),                                  # 576
-    (3585, 3457, 255, "x3_t64", 1), (3585, 3457, 256, "x3", 1),       # 812
+    (3585, 3457, 191, "x3_t64", 1), (3585, 3457, 192, "x3", 1),       # 812
+    (2049, 3079, 1025, "x3", 1), (2305, 2400, 1000, "x3", 1), (2305, 2300, 1000, "x3_t64", 1),  # 425, 361, 342
     (16, 32001, 1000, "x3_t64", 2), (150, 20000, 1500, "x3_t64", 1),  # 128 x 128 tiles mostly empty
 ])
 def test_fp32_tiles_and_ranges(m, n, k, kernel, ranges):

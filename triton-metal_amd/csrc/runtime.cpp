@@ -704,14 +704,16 @@ bool gemm_w4_enabled() {
  * with at most two 64 x 64 tiles per compute unit (below, the generic kernel: the
  * steps have nothing to overlap; 500^2, K = 64 5.4 us here and 5.0 there, 1000^2 6.2
  * and 5.6, 2001^2 11.2 and 12.0).
- * 128 x 128 or 64 x 64 tiles, us: the large ones where they come in three and more
- * rounds of one per compute unit, from K = 256 (2500 x 5000 in 800 tiles: K = 256 64
- * and 64, K = 1000 208 and 230; 6000^2, K = 512 257 and 313), and where half to all
- * of the compute units have one and a K past 900 splits into ranges (1001 x 2003 in
- * 128: K = 700 39.5 and 37.4, K = 2000 73.7 and 88; 2001^2 in 256: K = 700 59.5 and
- * 57.2, K = 2000 131 and 163).  Between, their second round is mostly empty (3001^2
- * in 576: K = 512 98 and 86, K = 4100 666 and 595).  Not where they cover a quarter
- * more than the small ones do (16 x 32001, K = 1000: 66.8 and 45.5). */
+ * 128 x 128 or 64 x 64 tiles, us: the large ones, two to a compute unit, where they
+ * fill seven tenths of their rounds, from K = 192 (2561 x 2500 in 420 tiles, 0.82 of
+ * a round, K = 300 44 and 46, K = 1000 122 and 136; 4097 x 3500 in 924, 0.90 of two,
+ * K = 200 61 and 64, K = 1000 225 and 266; 2401 x 2432 in 361, 0.71, K = 200 31 and 32,
+ * K = 2000 200 and 222; but 2100 x 2400 in 323, 0.63, K = 300 40 and 37, K = 2000 203
+ * and 203, and 3001^2 in 576, 0.56, K = 512 98 and 86); and where half to all of the
+ * compute units have one and a K past 900 splits into ranges (1001 x 2003 in 128: K =
+ * 700 39.5 and 37.4, K = 2000 73.7 and 88; 2001^2 in 256: K = 700 59.5 and 57.2, K =
+ * 2000 131 and 163).  Not where they cover a quarter more than the small ones do (16 x
+ * 32001, K = 1000: 66.8 and 45.5). */
 bool choose_gemm_x3(Plan &plan, TmGemmArgs &p, const char *family) {
   const bool gemm = strcmp(family, "gemm") == 0;
   if (!fast_paths_enabled() || p.scn != 1 || p.k <= 32) return false;
@@ -725,7 +727,8 @@ bool choose_gemm_x3(Plan &plan, TmGemmArgs &p, const char *family) {
   const int64_t large = cdiv(p.m, 128) * cdiv(p.n, 128), small = cdiv(p.m, 64) * cdiv(p.n, 64);
   if (p.k <= 64 && small <= 2 * cus) return false;
   const bool big = 16 * large <= 5 * small &&
-                   (large >= 3 * cus ? p.k >= 256 : large <= cus && 2 * large >= cus && p.k >= 900);
+                   (large > cus ? p.k >= 192 && 10 * large >= 7 * 2 * cus * cdiv(large, 2 * cus)
+                                : 2 * large >= cus && p.k >= 900);
   const int tile = big ? 128 : 64;
   plan.variant = format("tm_%s_x3%s%s_f32", family, b_t ? "_nt" : a_t ? "_tn" : "", big ? "" : "_t64");
   plan.grid[0] = (unsigned)(cdiv(p.m, tile) * cdiv(p.n, tile));
