@@ -41,7 +41,7 @@ def test_short_walks_and_larger_grids_take_two_waves(device, heads, seq):
 @pytest.mark.parametrize("causal", [False, True])
 @pytest.mark.parametrize("heads,seq,dim,pad,kept", [
     (2, 1, 80, 0, True), (3, 65, 65, 1, True), (6, 113, 80, 3, True), (2, 512, 72, 0, True),
-    (2, 513, 80, 0, True), (2, 100, 81, 0, True), (65, 128, 80, 0, False), (5, 513, 80, 0, False),
+    (2, 513, 80, 0, False), (2, 100, 81, 0, True), (65, 128, 80, 0, False),
 ])
 def test_fp32_forward_65_to_80(device, heads, seq, dim, pad, causal, kept):
     out, variants, dense, _ = _attention(heads, seq, dim, "f32", causal, stride_seq=dim + pad)
@@ -55,10 +55,10 @@ def test_fp32_forward_65_to_80(device, heads, seq, dim, pad, causal, kept):
 @pytest.mark.parametrize("heads,seq,dim,pad,kept", [
     # forward, dQ, dK/dV on the fp32 MFMAs
     (2, 97, 5, 2, "111"), (1, 1000, 20, 0, "111"), (6, 113, 40, 0, "111"),   # small, at most 40 columns
-    (2, 97, 41, 1, "100"), (3, 65, 88, 0, "101"), (2, 96, 103, 1, "101"),    # the forward, dK/dV past 64
+    (2, 97, 41, 1, "100"), (3, 65, 88, 0, "100"), (2, 96, 103, 1, "101"),    # the forward, dK/dV past 96
     (1, 129, 111, 1, "100"), (1, 129, 112, 0, "000"), (2, 96, 64, 0, "000"),
     (24, 300, 33, 0, "000"), (50, 150, 5, 2, "000"),                         # larger
-    (24, 300, 72, 4, "101"), (24, 300, 81, 1, "001"), (24, 300, 104, 0, "000"), (24, 300, 96, 0, "000"),
+    (24, 300, 72, 4, "100"), (24, 300, 81, 1, "000"), (24, 300, 100, 0, "001"), (24, 300, 104, 0, "000"), (24, 300, 96, 0, "000"),
 ])
 def test_fp32_kernels_by_head_dimension(device, heads, seq, dim, pad, causal, kept):
     out, variants, dense, _ = _attention(heads, seq, dim, "f32", causal, stride_seq=dim + pad)

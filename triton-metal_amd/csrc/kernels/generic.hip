@@ -234,5 +234,4 @@ TM_ATTN_MFMA32(DQ, 32)
 TM_ATTN_MFMA32(DQ, 64)
 TM_ATTN_MFMA32(DKDV, 32)
 TM_ATTN_MFMA32(DKDV, 64)
-TM_ATTN_MFMA32(DKDV, 96)
 TM_ATTN_MFMA32(DKDV, 128)

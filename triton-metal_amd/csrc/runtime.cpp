@@ -1095,8 +1095,9 @@ int64_t fast_ranges(int64_t wgs, int64_t n_ctx, int head_dim) {
  *    28.4; the forward of 2 heads of 96 at 88 columns 13.7 and 15.2, at 112 16.0 and 15.7;
  *  - the forward of 65 to 80 columns up to half the compute units and 512 keys: 16
  *    of 256 19.1 and 20.1, 4 of 512 17.9 and 19.1; 40 of 300 49.7 and 47.1;
- *  - dK/dV of 65 to 103 columns but 96, one wave per SIMD in the split form: 32 heads
- *    of 1000 at 80 columns 271 and 282, at 100 342 and 366, at 104 343 and 316. */
+ *  - dK/dV of 97 to 103 columns, one wave per SIMD in the split form: 32 heads of
+ *    1000 at 100 columns 342 and 366, at 104 343 and 316 (at 80 271 and 282, where the
+ *    split form's error is half: 3.9 and 2.0e-7). */
 enum class AttnOp { Fwd, Dq, Dkdv };
 bool attn_fp32_mfma(const BuiltinSpec &spec, AttnOp op, int64_t wgs, int64_t n_ctx) {
   const int d = spec.head_dim;
@@ -1104,10 +1105,10 @@ bool attn_fp32_mfma(const BuiltinSpec &spec, AttnOp op, int64_t wgs, int64_t n_c
   const bool short_grid = 2 * wgs <= device().compute_units, small = short_grid && wgs * n_ctx <= 20000;
   switch (op) {
     case AttnOp::Fwd:
-      return (small && d < 112) ||
+      return (small && d < 112 && (d <= 64 || d > 80)) ||
              (short_grid && d > 64 && d <= 80 && n_ctx <= 512);
     case AttnOp::Dq: return small && d <= 40;
-    case AttnOp::Dkdv: return (small && d <= 40) || (d > 64 && d < 104);
+    case AttnOp::Dkdv: return (small && d <= 40) || (d > 96 && d < 104);
   }
   return false;
 }
