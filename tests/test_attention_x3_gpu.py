@@ -1,6 +1,9 @@
 """fp32 attention on the bf16 matrix cores (three-way split operands): block and
-head-dimension edges, odd strides, and values that the split cannot hold, which
-the generic body computes, all at the fp32 tests' bounds."""
+head-dimension edges, odd strides, the smallest values, probabilities and score
+gradients, and values and scores past the range of the split, which the generic body
+computes, all at the fp32 tests' bounds.  (Small grids of head dimensions that are
+no multiple of 32 run the fp32 MFMAs: test_attention_small_grids_gpu.py has larger
+ones.)"""
 
 import math
 

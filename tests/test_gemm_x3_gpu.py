@@ -1,7 +1,8 @@
 """fp32 GEMM and SAE encoder on the bf16 matrix cores (three-way split): every
 layout and tile size, ragged and odd shapes, K ranges, against fp64 within the
-fp32 accumulation bound K 2^-24 (|A| |B|), which also holds for values that the
-split cannot represent (the fp32 fallback)."""
+fp32 accumulation bound K 2^-24 (|A| |B|), which also holds for the smallest values
+there are and for values and results past the range of the split (the fp32
+fallback); sums of few products within their last places."""
 
 import numpy as np
 import pytest
@@ -86,8 +87,8 @@ def test_x3_operands_of_whole_2_mib(device, m, n, k, layout):
 @pytest.mark.parametrize("layout", ["nn", "nt", "tn"])
 @pytest.mark.parametrize("scale", [2.0 ** -115, 2.0 ** -99, 2.0 ** 60, 2.0 ** 100])
 def test_x3_keeps_small_and_large_values(device, layout, scale):
-    """A near the bottom of the range (its low parts would be subnormal: the
-    fallback) and near the top, B such that the products stay in range."""
+    """A near the bottom of the range (its low parts subnormal but for the factor the
+    split gives them) and near the top, B such that the products stay in range."""
     rng = np.random.default_rng(2)
     m, n, k = 70, 90, 77
     a = (rng.standard_normal((m, k)) * scale).astype(np.float32)

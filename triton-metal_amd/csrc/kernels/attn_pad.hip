@@ -7,6 +7,8 @@
  * from 251 to 21.8 us, dQ from 285 to 24.1, dK/dV from 561 to 35.0.  What bounds
  * them is what bounds attn_fast.h's kernels, plus the columns between head_dim
  * and the contracted width (scores contract whole 32-column steps: 96 for 80).
+ * f16 holds P unscaled (PBias in attn_fast.h).  dQ and dK/dV of few heads run over
+ * ranges (attn_ranges.hip); the forward does not.
  */
 #include "attn_fast.h"
 

@@ -14,7 +14,8 @@
  * rows at 64 columns 204 / 239 / 306 and 172 / 190 / 231, at 128 columns 379 / 478
  * / 669 and 295 / 342 / 569; 2 heads of 96 11.7 / 12.8 / 16.4 and 10.1 / 10.6 /
  * 14.2 (six products, which lost bits: 160 / 168 / 207, 267 / 296 / 466 and 10.0 /
- * 9.9 / 14.1).  Beside the MFMAs there is the split (5.5 VALU
+ * 9.9 / 14.1).  The MFMA pipes are busy 34 / 45 / 49% of the time at 64 columns and
+ * 39 / 50 / 38% at 128; the rest is the split (5.5 VALU
  * operations an element and as much again for P and dS) and the LDS round trip
  * between a block's two barriers, which two or three workgroups per CU cover
  * in part.

@@ -87,7 +87,8 @@ TM_DEV int b_off(int row, int chunk) { return row * (2 * BN) + ((chunk ^ b_swz<B
 
 /* Each copy instruction moves a few whole rows of a tile through a buffer
  * resource based at its first row, whose range ends at the matrix's last
- * element (rounded up to 16 bytes, inside the allocation's 256-byte padding):
+ * element, rounded up to 16 bytes (rows are 16-byte aligned, so that stays inside
+ * the allocation, of whole 256 bytes):
  * rows past the last row of A or B are read as zeros, and a lane's byte
  * offset is the same for every instruction and k-step, so the addresses cost
  * only scalar instructions.  `rows_left` counts the valid rows from `base`,
@@ -171,8 +172,8 @@ TM_DEV void stage_b_global(const T *b, int64_t ldb, int k0, char *tile, int wave
  * element alignment (global memory takes them; a wave's 1 KB touches one more
  * cache line than an aligned one), issued at a step's start, written to the
  * next step's LDS tile (the same layouts) after its MFMAs.  Addresses stay
- * inside the operand and the 14 bytes after its last element, which its
- * allocation pads: a row of a K-contiguous tile (CONTIG) past the matrix
+ * inside the operand and the 14 bytes after its last element (the planner checks
+ * that its allocation has them): a row of a K-contiguous tile (CONTIG) past the matrix
  * repeats the last one and a chunk of a k-major tile past the last column the
  * last column's (both feed outputs that are not stored); in the last step the
  * chunks of a CONTIG tile past K start at K - 1 (the caller clears them) and

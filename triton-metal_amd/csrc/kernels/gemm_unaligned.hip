@@ -4,6 +4,7 @@
  * with register-staged tiles (UNAL).  tm_{gemm,sae}_generic_* are the 64 x 64-tile
  * ones of every layout, and the fp32-MFMA kernel (gemm_generic.h) for strides
  * that are not unit in either dimension: TmGemmArgs.layout says which.
+ * (Operands whose buffers have no 14 bytes behind them stay on that too.)
  * The fp32-MFMA kernel, which ran all of these before, converts every element
  * and contracts at a sixteenth of the 16-bit rate.  bf16, row-major, us before
  * and now: 2049 x 4097 x 1025 455 and 50, 4097 x 4099 x 4101 3346 and 264 (rows

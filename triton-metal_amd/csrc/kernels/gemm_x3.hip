@@ -10,10 +10,11 @@
  * to 1.41 off there.  Eight bf16 MFMAs take half the fp32 MFMA's time.
  *
  * Measured (us, fp32 MFMA kernels before and now): 2049 x 3079 x 1025 177 and
- * 110, 4096^3 1050 and 850, 1500^3 114 and 66, 1000^3 40 and 32, 129 x 202 x 7481
- * 276 and 27.  Beside the MFMAs there is what two workgroups per CU leave uncovered
- * of the split (6 VALU operations an element), the LDS writes and transposed reads
- * between its barriers.
+ * 111, 4096^3 1050 and 754 (182 TFLOP/s), 1500^3 121 and 75, 1000^3 43 and 31, 129 x
+ * 202 x 7481 273 and 29.  The MFMA pipes are busy 64% of the time at 4096^3, at the
+ * power limit's clock, and 42% at 2049 x 3079 x 1025, whose 425 tiles fill 0.83 of a
+ * round; the rest is what two workgroups per CU leave uncovered of the split (6 VALU
+ * operations an element), the LDS writes and transposed reads between its barriers.
  * Splitting into registers behind the MFMAs instead ran 93 / 738 us, three
  * workgroups per CU (168 registers) 114 / 818.
  *

@@ -4,10 +4,12 @@
  * LDS as f32 and contract on v_mfma_f32_16x16x4_f32, which multiplies exactly
  * for all three element types (gemm_generic.h, attn_generic.h).  What runs here:
  * 16-bit attention whose rows are not 16-byte aligned, whose head dimension is
- * no multiple of 8, or whose grid is tiny (ranges fill the chip); fp32 products
- * of at most 32 columns of K or of strides that are not 1; the range combines
- * and reduces; Delta.  (fp32 attention: attn_x3.hip, with these bodies as its
- * fallback.)  The reference's numerics:
+ * no multiple of 8, or whose grid is tiny, and the forward of one long head of few
+ * columns (ranges fill the chip); fp32 products of at most two 32-wide steps of K,
+ * of strides that are not 1, or of ragged sizes whose 16-byte loads have no room
+ * behind an operand; the range combines and reduces; Delta; fp32 attention of part
+ * of 32 columns where attn_x3.hip, whose fallback these bodies are, is slower.  The
+ * reference's numerics:
  *   - f32 accumulation everywhere (GEMMKernel.swift:46, AttentionKernel.swift:59-65);
  *   - P and dS rounded to the element type before the dot they feed
  *     (AttentionKernel.swift:59-65, AttentionBackwardKernel.swift:155-160, :357-369);

@@ -685,20 +685,6 @@ bool gemm_w4_enabled() {
 #define TM_GEMM_KSPLIT 1
 #endif
 
-/* Kernel choice shared by matmul_kernel and sae_encode_kernel.  The
- * specialised kernels take 16-bit elements and row-major operands with unit
- * inner stride, 16-byte aligned rows of A and B
- * and rows no shorter than the matrix (lda >= K, ldb >= N): whole tiles (K a
- * multiple of 64, 8-byte aligned rows of C) run the aligned kernel, any other
- * M, N, K the ragged one, whose copies clip at the matrix's last row and whose
- * last k-step and stores are masked.  Rows of A or B at other addresses run the
- * unaligned kernels, whose tiles go through registers (2049 x 4097 x 1025 bf16:
- * 50 us against 454 on the generic fp32-MFMA kernel).  Either operand (not both) may instead be stored
- * transposed: B with unit stride along K (the x @ W^T layout), read like A,
- * or A with unit stride along M (dY^T X), read like B.  fp32 with the same
- * layouts, 16-byte aligned rows and whole 128 x 128 (or, for problems with
- * few of those, 64 x 64) x 32 tiles runs the fp32 MFMA kernel.  Anything else
- * runs the generic 64 x 64 kernel. */
 /* fp32 on the bf16 matrix cores (gemm_x3.hip): any M, N, 4-byte aligned rows,
  * either operand (not both) stored transposed, K past one 32-wide step, past two
  * with at most two 64 x 64 tiles per compute unit (below, the generic kernel: the
@@ -736,6 +722,22 @@ bool choose_gemm_x3(Plan &plan, TmGemmArgs &p, const char *family) {
   return true;
 }
 
+/* Kernel choice shared by matmul_kernel and sae_encode_kernel.  The
+ * specialised kernels take 16-bit elements and row-major operands with unit
+ * inner stride, 16-byte aligned rows of A and B
+ * and rows no shorter than the matrix (lda >= K, ldb >= N): whole tiles (K a
+ * multiple of 64, 8-byte aligned rows of C) run the aligned kernel, any other
+ * M, N, K the ragged one, whose copies clip at the matrix's last row and whose
+ * last k-step and stores are masked.  Rows of A or B at other addresses run the
+ * unaligned kernels, whose tiles go through registers (2049 x 4097 x 1025 bf16:
+ * 50 us against 454 on the generic fp32-MFMA kernel).  Either operand (not both)
+ * may instead be stored transposed: B with unit stride along K (the x @ W^T
+ * layout), read like A, or A with unit stride along M (dY^T X), read like B.
+ * fp32 in the same layouts: whole 128 x 128 (or, for problems with few of those,
+ * 64 x 64) x 32 tiles of 16-byte aligned rows run the fp32 MFMA kernel or the
+ * bf16-split one, other sizes and rows at any 4-byte address the bf16-split one.
+ * `overhang`: 14 bytes can be read behind A and behind B, as rows at any address
+ * ask.  Anything else runs the generic 64 x 64 kernel. */
 void choose_gemm(Plan &plan, TmGemmArgs &p, const BuiltinSpec &spec, const char *family,
                  bool overhang) {
   const char *el = element_name(spec.element);

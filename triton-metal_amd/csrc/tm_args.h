@@ -18,11 +18,11 @@
 
 #include <stdint.h>
 
-/* which strides of A and B are 1: any, both inner ones (row-major), B's along K
- * (B stored transposed), A's along M (A stored transposed) */
 /* LDS of one K group of the 16-bit 64 x 64-tile kernels that take their groups
  * from the launch (twice it at 128 x 128; the generic any-stride body uses less) */
 #define TM_GEMM_GROUP_LDS 32768
+/* which strides of A and B are 1: any, both inner ones (row-major), B's along K
+ * (B stored transposed), A's along M (A stored transposed) */
 enum TmGemmLayout { TM_GEMM_ANY = 0, TM_GEMM_NN = 1, TM_GEMM_NT = 2, TM_GEMM_TN = 3 };
 
 struct TmGemmArgs {
@@ -86,8 +86,8 @@ struct TmAttnDqArgs {
   float sm_scale;
   int32_t stride_head, stride_seq, stride_lse, n_ctx;
   int32_t head_dim, heads;
-  /* key-range split (small grids, generic kernels): workgroup z walks the
-   * z-th of `splits` ranges of its key blocks and writes its unscaled fp32 dQ
+  /* key-range split (small grids, generic and _ranges kernels): workgroup z walks
+   * the z-th of `splits` ranges of its key blocks and writes its unscaled fp32 dQ
    * to part [splits][heads][n_ctx][head_dim], summed by tm_attn_split_reduce_* */
   float *part;
   int32_t splits;
@@ -105,8 +105,8 @@ struct TmAttnDkdvArgs {
   float sm_scale;
   int32_t stride_head, stride_seq, stride_lse, n_ctx;
   int32_t head_dim, heads;
-  /* query-range split (small grids, generic kernels): workgroup z walks the
-   * z-th of `splits` ranges of its query blocks and writes its unscaled fp32
+  /* query-range split (small grids, generic and _ranges kernels): workgroup z
+   * walks the z-th of `splits` ranges of its query blocks and writes its unscaled fp32
    * dK then dV to part [splits][2][heads][n_ctx][head_dim] */
   float *part;
   int32_t splits;
