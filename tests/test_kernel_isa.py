@@ -129,3 +129,12 @@ def test_gemm_and_sae_kernels_do_not_spill():
         for name, m in _meta(prefix).items():
             assert m[".vgpr_spill_count"] == 0 and m[".private_segment_fixed_size"] == 0, name
             assert m[".group_segment_fixed_size"] <= 160 * 1024, name
+
+
+def test_fp32_split_kernels_do_not_spill():
+    # two waves per SIMD (one for dK/dV past 64 columns)
+    for prefix in ("tm_gemm_x3_", "tm_sae_x3_", "tm_attn_fwd_generic_f32_d", "tm_attn_dq_generic_f32_d",
+                   "tm_attn_dkdv_generic_f32_d"):
+        for name, m in _meta(prefix).items():
+            assert m[".vgpr_spill_count"] == 0 and m[".private_segment_fixed_size"] == 0, name
+            assert m[".vgpr_count"] <= (512 if "dkdv" in name else 256), name
